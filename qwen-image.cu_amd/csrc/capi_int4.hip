@@ -137,7 +137,7 @@ int qimg_w4a4_gemm(const uint8_t* act_packed, const uint8_t* wgt_packed, const f
     QIMG_REQUIRE(all_aligned16(act_packed, wgt_packed, act_scales, wgt_scales, out),
                  "%s: pointers must be 16-byte aligned", fn);
     return api_hip_status(qimg::launch_w4a4_gemm(act_packed, wgt_packed, act_scales, wgt_scales, out, M, N, K,
-                                                 group_size, accumulate != 0, bias_bf16, 0, hs(stream)),
+                                                 group_size, accumulate != 0, bias_bf16, nullptr, nullptr, 0, 0, hs(stream)),
                           fn);
 }
 
@@ -189,6 +189,7 @@ int qimg_linear_int4(const float* x, int M, const qimg_int4_weight* w, const uin
         e = qimg::launch_int4_prep(x, w->smooth, xs, reinterpret_cast<uint16_t*>(base + L.xr), M, K, hbs, s);
     if (e != hipSuccess) return api_hip_status(e, fn);
     // 2. low-rank branch: lr = bf16(x_lr . svd_down), out = lr . svd_up^T
+    const bool fused = w4a4 && r > 0 && r % 16 == 0;  // the W4A4 kernel multiplies by svd_up itself
     if (r > 0) {
         uint16_t* svd_t = reinterpret_cast<uint16_t*>(base + L.svd_t);
         float* lr32 = reinterpret_cast<float*>(base + L.lr32);
@@ -196,13 +197,16 @@ int qimg_linear_int4(const float* x, int M, const qimg_int4_weight* w, const uin
         if ((e = qimg::launch_transpose_u16(w->svd_down, svd_t, K, r, s)) != hipSuccess ||
             (e = qimg::launch_linear_bf16(xs, QIMG_BF16, M, K, svd_t, r, nullptr, lr32, 0, s)) != hipSuccess ||
             (e = qimg::launch_f32_to_bf16(lr32, lr16, static_cast<int64_t>(M) * r, s)) != hipSuccess ||
-            (e = qimg::launch_linear_bf16(lr16, QIMG_BF16, M, r, w->svd_up, N, nullptr, out, 0, s)) != hipSuccess)
+            (!fused && (e = qimg::launch_linear_bf16(lr16, QIMG_BF16, M, r, w->svd_up, N, nullptr, out, 0, s)) !=
+                           hipSuccess))
             return api_hip_status(e, fn);
     }
     // 3. residual onto it, then the bias and GELU
     if (w4a4) {
         e = qimg::launch_w4a4_gemm(base + L.a, w->w4a4_qweight, reinterpret_cast<const float*>(base + L.act_scales),
-                                   w->w4a4_wscales, out, M, N, K, gs, r > 0, bias_bf16, gelu != 0, s);
+                                   w->w4a4_wscales, out, M, N, K, gs, r > 0 && !fused, bias_bf16,
+                                   fused ? reinterpret_cast<const uint16_t*>(base + L.lr16) : nullptr, w->svd_up, r,
+                                   gelu != 0, s);
     } else {
         uint16_t* deq = reinterpret_cast<uint16_t*>(base + L.a);
         e = nk16 ? qimg::launch_dequant_int4_bf16(w->qweight, w->scales4, deq, N, K, gs, 0, 1, 1, s)

@@ -158,176 +158,235 @@ __global__ __launch_bounds__(256) void quant_act_int4_kernel(const float* __rest
 }
 
 // ---- W4A4 GEMM ---------------------------------------------------------
-// A 512-thread workgroup owns a 128 x 128 output tile: eight waves in a 4 x 2
-// arrangement, each a 32 x 64 wave tile (two 32 x 32 blocks), two waves per
-// SIMD so that one wave's rescale (VALU work on every accumulator, each
-// group) runs beside the other's MFMAs. Operand chunks are loaded two chunks
-// ahead of their use, and the tile's scales of up to 64 groups at a time sit
-// in LDS: loading them from global memory inside each rescale left the
-// kernel waiting on their latency every group (290 -> 495 TOP/s at
-// 4096 x 3072 x 3072, group 64, bit-identical). Capping the registers at
-// 128 for four waves per SIMD spilled and ran at half the speed.
-constexpr int W4_THR = 512;
-constexpr int W4_BM = 128;
+// The kernel is bound by the vector ALU: each group of 64 columns costs a
+// 32 x 32 block two MFMAs (64 cycles of the matrix core) and 16 x 4 vector
+// operations (a conversion, two products and a sum per accumulator in the
+// reference's rounding order, 256 cycles). So everything else is kept off the
+// vector pipe's critical path: packed operands come by DMA into a two-slot
+// LDS ring of 128 columns (one barrier a stage), and the outputs are laid out
+// with n across the lanes, so a store writes 128 consecutive bytes of two rows
+// and the activation scales are LDS broadcasts. A wave owns 32 x 64 outputs
+// (four waves per SIMD); 64 x 64 (two per SIMD, fewer unpacks per product)
+// measured 134 against 112 us at 4352 x 3072 x 3072, group 64, and 48 against
+// 30 us at 256 rows. Before, lanes ran across m (each 4-byte access touched
+// 64 lines) and fragments were loaded straight from global memory: 254 us, and
+// 19 us more for the low-rank product that is now multiplied here. 112 us is
+// 0.73 POP/s; the vector operations alone take about 92 us.
+constexpr int W4_THR = 256;   // four waves, 2 x 2
+constexpr int W4_BM = 64;
 constexpr int W4_BN = 128;
+constexpr int W4_STG = 64;    // packed bytes of a row per stage (128 columns)
 
 // Eight packed bytes (16 nibbles) -> one i8 MFMA fragment of 16 bytes, each
 // 16 x its signed nibble.
-__device__ __forceinline__ v4i unpack16(uint2 p) {
-    return (v4i){static_cast<int>((p.x << 4) & 0xF0F0F0F0u), static_cast<int>(p.x & 0xF0F0F0F0u),
-                 static_cast<int>((p.y << 4) & 0xF0F0F0F0u), static_cast<int>(p.y & 0xF0F0F0F0u)};
+__device__ __forceinline__ v4i unpack16(uint32_t x, uint32_t y) {
+    return (v4i){static_cast<int>((x << 4) & 0xF0F0F0F0u), static_cast<int>(x & 0xF0F0F0F0u),
+                 static_cast<int>((y << 4) & 0xF0F0F0F0u), static_cast<int>(y & 0xF0F0F0F0u)};
 }
 
-// out[m,n] (+)= sum_g ((float)d_g * as[g,m]) * ws[g,n] + bias[n] (then GELU,
-// gelu_fp32 after the reference's GEMM, cuda_kernels.cu:4529-4531). The MFMA
-// is issued as D = W x A^T, so lane l holds m = l % 32 and n rows
-// 8 (r/4) + 4 (l/32) + r%4 of each 32 x 32 block. gs % 64 == 0.
-__global__ __launch_bounds__(W4_THR) void w4a4_gemm_kernel(const uint8_t* __restrict__ act,
-                                                           const uint8_t* __restrict__ wgt,
-                                                           const float* __restrict__ as,
-                                                           const float* __restrict__ ws, float* out, int M, int N,
-                                                           int K, int gs, int accumulate,
-                                                           const uint16_t* __restrict__ bias, int gelu) {
+// out[m,n] = sum_g ((float)d_g * as[g,m]) * ws[g,n] + bias[n], onto the
+// low-rank product lr[m,:] . up[n,:] (bf16 factors of rank r, r % 16 == 0,
+// fp32 sums; the reference adds the residual to it, cuda_kernels.cu:4521) or,
+// with `accumulate`, onto out's own values; then GELU (gelu_fp32,
+// :4529-4531). CH: 64-column chunks of a group (0: any number). The MFMA is issued as D = A x W^T: lane l holds column
+// n = l % 32 and rows m = 8 (r/4) + 4 (l/32) + r%4 of each 32 x 32 block.
+template <int CH, bool GELU>
+__global__ __launch_bounds__(W4_THR) void w4a4_gemm_kernel(const uint8_t* act,
+                                                              const uint8_t* wgt,
+                                                              const float* as,
+                                                              const float* ws, float* out, int M, int N,
+                                                              int K, int chunks, int accumulate,
+                                                              const uint16_t* bias,
+                                                              const uint16_t* lr,
+                                                              const uint16_t* up, int r) {
+    constexpr int NDMA = (W4_BM + W4_BN) / 16 / (W4_THR / 64);  // DMA instructions per wave and stage
+    // One LDS object: with a second one, or with restrict arguments, the
+    // compiler holds every LDS read until the DMA in flight has landed.
+    constexpr int OPB = (W4_BM + W4_BN) * W4_STG;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * OPB + 4 * (W4_BM + W4_BN) * 4];
+    float (*s_sc)[2][W4_BM + W4_BN] = reinterpret_cast<float (*)[2][W4_BM + W4_BN]>(lds + 2 * OPB);
     const int tiles_m = (M + W4_BM - 1) / W4_BM;
     const int tiles_n = (N + W4_BN - 1) / W4_BN;
     const int logical = xcd_remap(blockIdx.x, tiles_m * tiles_n);
     // M-tile fastest: consecutive workgroups share a weight slice
     const int m0 = (logical % tiles_m) * W4_BM;
     const int n0 = (logical / tiles_m) * W4_BN;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int h = lane >> 5;
     const int KB = K / 2;
-    const int G = K / gs;
+    const int nch = K / 64;
+    const int nst = (nch + 1) / 2;
 
-    const int m = m0 + wm * 32 + (lane & 31);
-    const int mrow = m < M ? m : M - 1;  // rows past the end are computed, never stored
-    // Lane half h takes packed bytes [16h, 16h + 16) of each 32-byte
-    // (64-column) chunk of its row, one 16-byte load for two MFMA steps:
-    // bytes 16h + 8s .. +8 feed step s (a k order that both operands share).
-    const uint8_t* ap = act + static_cast<int64_t>(mrow) * KB + 16 * h;
-    const uint8_t* wp[2];
-    int ncol[2][4];  // the 16 output columns of block j held by this lane, as 4 runs of 4
+    // A DMA instruction fills 16 rows x 64 bytes. Chunk c (16 bytes) of row t
+    // sits at position c ^ ((t >> 2) & 3), so the 16 rows of a fragment read
+    // cover all banks. Rows past the end repeat the last one (computed,
+    // never stored); the half stage past an odd number of chunks repeats
+    // the row's start (never used).
+    const uint8_t* src[NDMA];
+    int col[NDMA];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int n = n0 + wn * 64 + 32 * j + (lane & 31);
-        wp[j] = wgt + static_cast<int64_t>(n < N ? n : N - 1) * KB + 16 * h;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) ncol[j][q] = n0 + wn * 64 + 32 * j + 8 * q + 4 * h;
+    for (int i = 0; i < NDMA; ++i) {
+        const int t = (wave * NDMA + i) * 16 + (lane >> 2);
+        col[i] = 16 * ((lane & 3) ^ ((t >> 2) & 3));
+        const bool is_a = t < W4_BM;
+        const int row = is_a ? m0 + t : n0 + t - W4_BM;
+        const int last = (is_a ? M : N) - 1;
+        src[i] = (is_a ? act : wgt) + static_cast<int64_t>(row < last ? row : last) * KB;
     }
+    auto issue = [&](int st, int slot) {
+#pragma unroll
+        for (int i = 0; i < NDMA; ++i) {
+            const int c = st * W4_STG + col[i];
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src[i] + (c < KB ? c : 0)),
+                                             (lds_ptr_t)(lds + slot * OPB + (wave * NDMA + i) * 1024), 16, 0, 1);
+        }
+    };
+    // The scales of a stage's two chunks: thread t carries row t's (as, times
+    // the 2^-8 of the unpacking) or column t - W4_BM's.
+    const bool sc_a = tid < W4_BM;
+    const bool sc_live = tid < W4_BM + W4_BN;
+    const int sc_i = sc_a ? (m0 + tid < M ? m0 + tid : M - 1) : (n0 + tid - W4_BM < N ? n0 + tid - W4_BM : N - 1);
+    const int sc_stride = sc_a ? M : N;
+    const float* sc_p = (sc_a ? as : ws) + sc_i;
+    const float sc_mul = sc_a ? 0.00390625f : 1.0f;
+    float sc[2] = {0.0f, 0.0f};
+    auto load_sc = [&](int st) {
+        if (!sc_live) return;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int c = 2 * st + u < nch ? 2 * st + u : nch - 1;
+            sc[u] = sc_p[static_cast<int64_t>(CH == 1 ? c : c / (CH ? CH : chunks)) * sc_stride];
+        }
+    };
+    auto store_sc = [&](int slot) {
+        if (!sc_live) return;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) s_sc[slot][u][tid] = sc[u] * sc_mul;
+    };
 
     float acc[2][16];
+    v16i d[CH == 0 ? 2 : 1];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+        for (int e = 0; e < 16; ++e) acc[j][e] = 0.0f;
 
-    const int chunks = gs / 64;  // 64-column chunks (two MFMA steps) per group
-    const int nch = K / 64;
-    // Chunk loads run PF chunks ahead of their use (the loads of a chunk
-    // are three 16-byte loads per lane straight from global memory).
-    constexpr int PF = 2;
-    uint4 ra[PF + 1], rw[PF + 1][2];
-    auto load = [&](int c, int slot) {
-        const int off = 32 * c;
-        ra[slot] = *reinterpret_cast<const uint4*>(ap + off);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) rw[slot][j] = *reinterpret_cast<const uint4*>(wp[j] + off);
+    auto mfma2 = [&](const u32x4& a, const u32x4& w, v16i c) {
+        c = __builtin_amdgcn_mfma_i32_32x32x32_i8(unpack16(a.x, a.y), unpack16(w.x, w.y), c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_i32_32x32x32_i8(unpack16(a.z, a.w), unpack16(w.z, w.w), c, 0, 0, 0);
     };
+    // (float)(d >> 8) * sa == (float)d * (sa * 2^-8): d = 256 x an exact sum
+    // below 2^24 in magnitude, and the power-of-two scaling is exact, so the
+    // product rounds identically.
+    auto rescale = [&](const v16i& dd, float (&o)[16], const float* s_a, float sw) {
 #pragma unroll
-    for (int p = 0; p < PF; ++p)
-        if (p < nch) load(p, p);
-    v16i d[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) d[j][r] = 0;
-    // The tile's activation and weight scales of up to SG groups at a time
-    // in LDS (loaded together between two barriers at a group boundary), so
-    // a group's rescale reads them without global latency.
-    constexpr int SG = 64;
-    __shared__ __attribute__((aligned(16))) float s_as[SG][W4_BM];
-    __shared__ __attribute__((aligned(16))) float s_ws[SG][W4_BN];
-    auto stage_scales = [&](int g0) {
-        const int ng = G - g0 < SG ? G - g0 : SG;
-        __syncthreads();  // every wave is done with the previous groups' scales
-        for (int i = threadIdx.x; i < ng * W4_BM; i += W4_THR) {
-            const int gi = i / W4_BM, r = i % W4_BM;
-            const int mm = m0 + r < M ? m0 + r : M - 1;
-            const int nn = n0 + r < N ? n0 + r : N - 1;
-            s_as[gi][r] = as[static_cast<int64_t>(g0 + gi) * M + mm] * 0.00390625f;
-            s_ws[gi][r] = ws[static_cast<int64_t>(g0 + gi) * N + nn];
-        }
-        __syncthreads();
-    };
-    const int mloc = wm * 32 + (lane & 31);
-    int g = 0, cg = 0;
-    stage_scales(0);
-    for (int c0 = 0; c0 < nch; c0 += PF + 1) {
-#pragma unroll
-        for (int u = 0; u < PF + 1; ++u) {
-            const int c = c0 + u;
-            if (c >= nch) break;
-            // slot of chunk c is u; chunk c + PF goes to slot (u + PF) % (PF + 1)
-            if (c + PF < nch) load(c + PF, (u + PF) % (PF + 1));
-            const uint4 pa = ra[u];
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const v4i fa = unpack16(s ? make_uint2(pa.z, pa.w) : make_uint2(pa.x, pa.y));
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const v4i fw = unpack16(s ? make_uint2(rw[u][j].z, rw[u][j].w) : make_uint2(rw[u][j].x, rw[u][j].y));
-                    // a group's first step starts from zero (no reset of d)
-                    const v16i zero = {};
-                    d[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw, fa, (s == 0 && cg == 0) ? zero : d[j], 0, 0, 0);
-                }
-            }
-            if (++cg == chunks) {
-                cg = 0;
-                // (float)(d >> 8) * sa == (float)d * (sa * 2^-8): d = 256 x an
-                // exact sum below 2^12 in magnitude, and the power-of-two
-                // scaling is exact, so the product rounds identically.
-                const int gi = g % SG;
-                const float sa = s_as[gi][mloc];
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const v4f sw = *reinterpret_cast<const v4f*>(&s_ws[gi][ncol[j][q] - n0]);
-#pragma unroll
-                        for (int cc = 0; cc < 4; ++cc) {
-#pragma clang fp contract(off)
-                            const float t = static_cast<float>(d[j][4 * q + cc]) * sa;
-                            acc[j][4 * q + cc] = acc[j][4 * q + cc] + t * sw[cc];
-                        }
-                    }
-                ++g;
-                if (g % SG == 0 && g < G) stage_scales(g);
-            }
-        }
-    }
-
-    if (m >= M) return;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 4; ++q) {
+            const v4f sa = *reinterpret_cast<const v4f*>(s_a + 8 * q);
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                const int n = ncol[j][q] + c;
-                if (n >= N) continue;
-                const float b = bias != nullptr ? bf16_to_f32(bias[n]) : 0.0f;
-                float* o = out + static_cast<int64_t>(m) * N + n;
-                float v;
-                {
 #pragma clang fp contract(off)
-                    v = acc[j][4 * q + c] + b;
-                    if (accumulate) v = *o + v;
-                }
-                if (gelu) v = gelu_tanh(v);
-                *o = v;
+                const float t = static_cast<float>(dd[4 * q + c]) * sa[c];
+                o[4 * q + c] = o[4 * q + c] + t * sw;
             }
+        }
+    };
+    const int arow = wm * 32 + (lane & 31);
+    const int wrow = wn * 64 + (lane & 31);
+    const int sw8 = ((lane & 31) >> 2) & 3;  // rows 32 apart share it
+
+    issue(0, 0);
+    load_sc(0);
+    store_sc(0);
+    int cg = 0;
+    for (int st = 0; st < nst; ++st) {
+        const int slot = st & 1;
+        wait_vmcnt<0>();  // this wave's part of the stage, issued a stage ago
+        wait_lgkmcnt0();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (st + 1 < nst) {
+            issue(st + 1, slot ^ 1);
+            load_sc(st + 1);
+        }
+        const uint8_t* ob = lds + slot * OPB;
+        if constexpr (CH == 2) {
+            u32x4 a[2], w[2][2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int off = 16 * ((2 * u + h) ^ sw8);
+                a[u] = *reinterpret_cast<const u32x4*>(ob + arow * W4_STG + off);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    w[j][u] = *reinterpret_cast<const u32x4*>(ob + (W4_BM + wrow + 32 * j) * W4_STG + off);
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const v16i zero = {};
+                const v16i dd = mfma2(a[1], w[j][1], mfma2(a[0], w[j][0], zero));
+                rescale(dd, acc[j], &s_sc[slot][0][wm * 32 + 4 * h], s_sc[slot][0][W4_BM + wrow + 32 * j]);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                if (2 * st + u >= nch) break;
+                const int off = 16 * ((2 * u + h) ^ sw8);
+                const u32x4 a = *reinterpret_cast<const u32x4*>(ob + arow * W4_STG + off);
+                u32x4 w[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    w[j] = *reinterpret_cast<const u32x4*>(ob + (W4_BM + wrow + 32 * j) * W4_STG + off);
+                const bool first = CH == 1 || cg == 0;
+                const bool last = CH == 1 || cg + 1 == chunks;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const v16i zero = {};
+                    v16i& dd = d[CH == 0 ? j : 0];
+                    dd = mfma2(a, w[j], first ? zero : dd);
+                    if (last)
+                        rescale(dd, acc[j], &s_sc[slot][u][wm * 32 + 4 * h], s_sc[slot][u][W4_BM + wrow + 32 * j]);
+                }
+                cg = last ? 0 : cg + 1;
+            }
+        }
+        if (st + 1 < nst) store_sc(slot ^ 1);
+    }
+
+    typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+    const int mb = m0 + wm * 32;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int n = n0 + wrow + 32 * j;
+        v16f low;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) low[e] = 0.0f;
+        if (lr != nullptr) {
+            const int ml = mb + (lane & 31) < M ? mb + (lane & 31) : M - 1;
+            const uint16_t* pl = lr + static_cast<int64_t>(ml) * r + 8 * h;
+            const uint16_t* pu = up + static_cast<int64_t>(n < N ? n : N - 1) * r + 8 * h;
+            for (int k = 0; k < r; k += 16)
+                low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const v8bf*>(pl + k),
+                                                              *reinterpret_cast<const v8bf*>(pu + k), low, 0, 0, 0);
+        }
+        if (n >= N) continue;
+        const float b = bias != nullptr ? bf16_to_f32(bias[n]) : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int m = mb + 8 * (e >> 2) + 4 * h + (e & 3);
+            if (m >= M) continue;
+            float* o = out + static_cast<int64_t>(m) * N + n;
+            float v;
+            {
+#pragma clang fp contract(off)
+                v = acc[j][e] + b;
+                if (lr != nullptr) v = low[e] + v;
+                if (accumulate) v = *o + v;
+            }
+            *o = GELU ? gelu_tanh(v) : v;
+        }
+    }
 }
 
 // ---- AWQ ----------------------------------------------------------------
@@ -583,15 +642,28 @@ hipError_t launch_quant_act_int4(const float* x, const float* smooth, uint16_t* 
     return hipGetLastError();
 }
 
+template <int CH>
+static void run_w4a4(unsigned tiles, const uint8_t* act, const uint8_t* wgt, const float* as, const float* ws, float* out,
+                     int M, int N, int K, int gs, int accumulate, const uint16_t* bias, const uint16_t* lr,
+                     const uint16_t* up, int r, int gelu, hipStream_t stream) {
+    if (gelu)
+        hipLaunchKernelGGL((w4a4_gemm_kernel<CH, true>), dim3(tiles), dim3(W4_THR), 0, stream, act, wgt, as, ws, out,
+                           M, N, K, gs / 64, accumulate, bias, lr, up, r);
+    else
+        hipLaunchKernelGGL((w4a4_gemm_kernel<CH, false>), dim3(tiles), dim3(W4_THR), 0, stream, act, wgt, as, ws, out,
+                           M, N, K, gs / 64, accumulate, bias, lr, up, r);
+}
+
 hipError_t launch_w4a4_gemm(const uint8_t* act, const uint8_t* wgt, const float* as, const float* ws, float* out,
-                            int M, int N, int K, int gs, int accumulate, const uint16_t* bias, int gelu,
-                            hipStream_t stream) {
+                            int M, int N, int K, int gs, int accumulate, const uint16_t* bias, const uint16_t* lr,
+                            const uint16_t* up, int r, int gelu, hipStream_t stream) {
     if (M == 0 || N == 0) return hipSuccess;
-    if (gs <= 0 || gs % 64 != 0 || K % gs != 0) return hipErrorInvalidValue;
+    if (gs <= 0 || gs % 64 != 0 || K % gs != 0 || (lr != nullptr && (up == nullptr || r <= 0 || r % 16 != 0)))
+        return hipErrorInvalidValue;
     const int64_t tiles = static_cast<int64_t>((M + W4_BM - 1) / W4_BM) * ((N + W4_BN - 1) / W4_BN);
     if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(w4a4_gemm_kernel, dim3(static_cast<unsigned>(tiles)), dim3(W4_THR), 0, stream, act, wgt, as, ws,
-                       out, M, N, K, gs, accumulate, bias, gelu);
+    auto* run = gs == 64 ? run_w4a4<1> : gs == 128 ? run_w4a4<2> : run_w4a4<0>;
+    run(static_cast<unsigned>(tiles), act, wgt, as, ws, out, M, N, K, gs, accumulate, bias, lr, up, r, gelu, stream);
     return hipGetLastError();
 }
 

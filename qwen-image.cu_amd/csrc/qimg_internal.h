@@ -142,9 +142,11 @@ hipError_t launch_quant_int4_weight(const float* r, uint8_t* qw, float* scales, 
                                     hipStream_t stream);
 hipError_t launch_quant_act_int4(const float* x, const float* smooth, uint16_t* bf16_out, uint8_t* packed,
                                  float* scales, int M, int K, int gs, hipStream_t stream);
+// lr / up non-null (r % 16 == 0): the result is added to the low-rank product
+// lr [M, r] . up [N, r]^T (bf16), computed in the same kernel.
 hipError_t launch_w4a4_gemm(const uint8_t* act, const uint8_t* wgt, const float* as, const float* ws, float* out,
-                            int M, int N, int K, int gs, int accumulate, const uint16_t* bias, int gelu,
-                            hipStream_t stream);
+                            int M, int N, int K, int gs, int accumulate, const uint16_t* bias, const uint16_t* lr,
+                            const uint16_t* up, int r, int gelu, hipStream_t stream);
 hipError_t launch_awq_repack(const int32_t* qw, int32_t* out, int OC, int IC, hipStream_t stream);
 hipError_t launch_awq_dequant(const int32_t* qw, const uint16_t* wscales, const uint16_t* wzeros, uint16_t* out,
                               int OC, int IC, int gs, int ncomp, hipStream_t stream);

@@ -110,6 +110,27 @@ def test_w4a4_gemm_bit_exact(qimg, oracle, M, N, K, gs, accumulate):
         np.testing.assert_array_equal(g[m:m + 1], want)
 
 
+@pytest.mark.parametrize("M,N,K,gs", [(65, 129, 192, 64), (63, 127, 576, 192), (64, 128, 320, 64), (2, 260, 64, 64),
+                                      (129, 64, 768, 256)])
+def test_w4a4_gemm_tile_edges_bit_exact(qimg, oracle, M, N, K, gs):
+    """An odd number of 64-column chunks (a half-filled last stage), groups of
+    three and four chunks, and rows and columns one past a tile."""
+    rng = np.random.default_rng(M + N + K)
+    ap = rng.integers(0, 256, (M, K // 2)).astype(np.uint8)
+    wp = rng.integers(0, 256, (N, K // 2)).astype(np.uint8)
+    asc = rng.uniform(0.001, 0.5, (K // gs, M)).astype(np.float32)
+    wsc = rng.uniform(0.001, 0.05, (K // gs, N)).astype(np.float32)
+    got = qimg.w4a4_gemm(_u8(ap), _u8(wp), _f32(asc), _f32(wsc), K, gs)
+    np.testing.assert_array_equal(got.cpu().numpy(), oracle.w4a4_gemm(ap, wp, asc, wsc, K, gs))
+
+
+@pytest.mark.parametrize("M,N,K,r,gs", [(65, 130, 320, 48, 64), (33, 100, 256, 16, 128), (33, 100, 256, 24, 64)])
+def test_linear_w4a4_low_rank(qimg, oracle, M, N, K, r, gs):
+    """The low-rank product inside the W4A4 kernel (ranks of 16, ragged tiles),
+    and a rank it does not take."""
+    test_linear_int4(qimg, oracle, M, N, K, r, gs, True, True, True, 1, r == 24)
+
+
 def test_awq_paths_bit_exact(qimg, oracle):
     rng = np.random.default_rng(2)
     OC, IC, gs, nc = 18432, 3072, 64, 6   # the modulation layer (6 x 3072 outputs)
