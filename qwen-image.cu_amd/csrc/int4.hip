@@ -435,54 +435,143 @@ __global__ __launch_bounds__(256) void awq_dequant_kernel(const int32_t* __restr
     }
 }
 
-// awq_gemv_repacked_kernel (cuda_kernels.cu:3106-3153), M = 1, gs = 64: one
-// lane per interleaved output channel, the input row in LDS, the sum over
-// ic in order (a dependent chain per lane). The next group's eight weight
-// words and its scale and zero are loaded while the current group is
-// summed, so the chain waits on the memory latency once, not per group;
-// 64-lane workgroups spread the channels over the CUs.
-__global__ __launch_bounds__(64) void awq_gemv_kernel(const float* __restrict__ x, const int32_t* __restrict__ qw,
-                                                      const uint16_t* __restrict__ wscales,
-                                                      const uint16_t* __restrict__ wzeros,
-                                                      const uint16_t* __restrict__ bias, float* __restrict__ out,
-                                                      int OC, int IC, int ncomp) {
-    extern __shared__ float s_x[];
-    for (int i = threadIdx.x; i < IC; i += blockDim.x) s_x[i] = x[i];
-    __syncthreads();
-    const int nk_raw = blockIdx.x * blockDim.x + threadIdx.x;
+// awq_gemv_repacked_kernel (cuda_kernels.cu:3106-3153), M = 1, gs = 64. The
+// sum over ic runs in order, so each output channel is one dependent chain of
+// IC additions, and a wave cannot issue a dependent addition before 8.4 cycles
+// have passed: 3072 of them are 11 us. Everything else is taken off that chain.
+// A workgroup owns 64 channels, one per lane: eight waves load the weight words
+// AWQ_DEPTH stages ahead, form the products and put them in a two-slot LDS
+// ring of 128 inputs; a ninth wave, first in the issue order, reads them (16
+// bytes a lane, the next 32 inputs while it adds the last) and adds. q * s is exact in fp32 (4 bits x a
+// bf16's 8), so fma(q, s, z) is the reference's q * s + z.
+// 18432 x 3072 (32 MB of weights and scales): 22.4 us; one wave per 64 channels
+// doing all of it took 74.6. With x in scalar registers, whose load latency
+// falls on every stage's barrier, 32.7; with the last sums' operands read in
+// one go (134 registers, so that two workgroups do not share a CU), 36.
+constexpr int AWQ_PW = 8;     // producer waves
+constexpr int AWQ_DEPTH = 4;  // stages of weight words in flight per producer
+constexpr int AWQ_THR = 64 * (AWQ_PW + 1);
+constexpr int AWQ_RING = 2 * 32 * 64;  // [slot][4 inputs][channel], 16 bytes each
+
+__global__ __launch_bounds__(AWQ_THR, 5) void awq_gemv_kernel(const float* __restrict__ x, const int32_t* __restrict__ qw,
+                                                           const uint16_t* __restrict__ wscales,
+                                                           const uint16_t* __restrict__ wzeros,
+                                                           const uint16_t* __restrict__ bias, float* __restrict__ out,
+                                                           int OC, int IC, int ncomp) {
+    constexpr int WPP = 16 / AWQ_PW;  // words of 8 inputs per producer and stage
+    extern __shared__ __attribute__((aligned(16))) v4f awq_lds[];  // the ring, then x
+    v4f* sx = awq_lds + AWQ_RING;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nk_raw = blockIdx.x * 64 + lane;
     const bool live = nk_raw < OC;
     const int nk = live ? nk_raw : OC - 1;
     const int G = IC / 64;
-    auto load = [&](int g, uint32_t* p, uint16_t& s, uint16_t& z) {
-#pragma unroll
-        for (int io = 0; io < 8; ++io) p[io] = static_cast<uint32_t>(qw[static_cast<int64_t>(g * 8 + io) * OC + nk]);
-        s = wscales[static_cast<int64_t>(g) * OC + nk];
-        z = wzeros[static_cast<int64_t>(g) * OC + nk];
+    // Stages in whole rounds of AWQ_DEPTH, so that the producers' loop has no
+    // exit inside a round and the loads in flight are counted exactly.
+    const int nst = ((G + 1) / 2 + AWQ_DEPTH - 1) / AWQ_DEPTH * AWQ_DEPTH;
+    // one barrier a stage: slot st & 1 is full, and the other one is read
+    auto stage_barrier = [] {
+        wait_lgkmcnt0();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
     };
-    uint32_t p[8], pn[8];
-    uint16_t s16, z16, sn16 = 0, zn16 = 0;
-    load(0, p, s16, z16);
-    float acc = 0.0f;
-    for (int g = 0; g < G; ++g) {
-        if (g + 1 < G) load(g + 1, pn, sn16, zn16);
-        const float s = bf16_to_f32(s16);
-        const float z = bf16_to_f32(z16);
-        const v4f* xv = reinterpret_cast<const v4f*>(s_x + g * 64);
+    if (wave < AWQ_PW) {
+        const int w0 = wave * WPP;  // first of the stage's 16 words
+        uint32_t q[AWQ_DEPTH][WPP];
+        uint16_t s16[AWQ_DEPTH], z16[AWQ_DEPTH];
+        // Stages past the end (and the half stage past an odd G) read the
+        // last group again; its products are never added.
+        auto group_of = [&](int st) {
+            const int g = 2 * st + (w0 >> 3);
+            return g < G ? g : G - 1;
+        };
+        auto load = [&](int d, int st) {
+            const int g = group_of(st);
+            const int32_t* p = qw + static_cast<int64_t>(g * 8 + (w0 & 7)) * OC + nk;
 #pragma unroll
-        for (int io = 0; io < 8; ++io) {
-            const v4f x0 = xv[2 * io], x1 = xv[2 * io + 1];
-            const float xs[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+            for (int i = 0; i < WPP; ++i) q[d][i] = static_cast<uint32_t>(p[static_cast<int64_t>(i) * OC]);
+            s16[d] = wscales[static_cast<int64_t>(g) * OC + nk];
+            z16[d] = wzeros[static_cast<int64_t>(g) * OC + nk];
+        };
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-#pragma clang fp contract(off)
-                const float w = static_cast<float>((p[io] >> (4 * k)) & 0xF) * s + z;
-                acc = acc + w * xs[k];
+        for (int d = 0; d < AWQ_DEPTH; ++d) load(d, d);
+        stage_barrier();  // x is in LDS
+        v4f xs[2 * WPP];
+        auto load_x = [&](int st) {
+            const v4f* xg = sx + group_of(st) * 16 + (w0 & 7) * 2;
+#pragma unroll
+            for (int i = 0; i < 2 * WPP; ++i) xs[i] = xg[i];
+        };
+        load_x(0);
+        for (int st0 = 0; st0 < nst; st0 += AWQ_DEPTH) {
+#pragma unroll
+            for (int d = 0; d < AWQ_DEPTH; ++d) {
+                const int st = st0 + d;
+                v4f v[2 * WPP];
+                const float s = bf16_to_f32(s16[d]), z = bf16_to_f32(z16[d]);
+#pragma unroll
+                for (int i = 0; i < WPP; ++i) {
+                    const uint32_t ev = q[d][i] & 0x0F0F0F0Fu, od = (q[d][i] >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const float n = static_cast<float>(((k & 1 ? od : ev) >> (8 * (k >> 1))) & 0xFFu);
+                        v[2 * i + (k >> 2)][k & 3] = __builtin_fmaf(n, s, z) * xs[2 * i + (k >> 2)][k & 3];
+                    }
+                }
+                load(d, st + AWQ_DEPTH);
+                v4f* ring = awq_lds + (st & 1) * (AWQ_RING / 2) + 2 * w0 * 64 + lane;
+#pragma unroll
+                for (int i = 0; i < 2 * WPP; ++i) ring[i * 64] = v[i];
+                load_x(st + 1);
+                stage_barrier();
             }
         }
+        return;
+    }
+    for (int i = lane; i < IC / 4; i += 64) sx[i] = reinterpret_cast<const v4f*>(x)[i];
+    stage_barrier();
+    __builtin_amdgcn_s_setprio(3);
+    float acc = 0.0f;
+    v4f va[8], vb[8];
 #pragma unroll
-        for (int io = 0; io < 8; ++io) p[io] = pn[io];
-        s16 = sn16;
-        z16 = zn16;
+    for (int c = 0; c < 8; ++c) vb[c] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    auto read = [&](v4f (&v)[8], int st, int u) {
+        const v4f* p = awq_lds + (st & 1) * (AWQ_RING / 2) + 8 * u * 64 + lane;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) v[c] = p[c * 64];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add = [&](const v4f (&v)[8]) {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = acc + v[c][e];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int st = 0;
+    for (; st < G / 2; ++st) {
+        stage_barrier();
+        read(va, st, 0);
+        add(vb);  // the last stage's last quarter (zeros at first)
+        read(vb, st, 1);
+        add(va);
+        read(va, st, 2);
+        add(vb);
+        read(vb, st, 3);
+        add(va);
+    }
+    add(vb);
+    for (; st < nst; ++st) {
+        stage_barrier();
+        if (2 * st < G) {  // the last of an odd number of groups
+            read(va, st, 0);
+            read(vb, st, 1);
+            add(va);
+            add(vb);
+        }
     }
     if (!live) return;
     const int dim = OC / ncomp;
@@ -689,8 +778,12 @@ hipError_t launch_awq_gemv(const float* x, const int32_t* qw_rep, const uint16_t
     if (OC == 0) return hipSuccess;
     // the reference's GEMV reads 8 words (64 inputs) per group
     if (gs != 64 || IC % 64 != 0 || ncomp <= 0 || OC % ncomp != 0 || IC > 16384) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(awq_gemv_kernel, dim3((OC + 63) / 64), dim3(64), IC * sizeof(float), stream, x, qw_rep, wscales,
-                       wzeros, bias, out, OC, IC, ncomp);
+    const int lds = AWQ_RING * 16 + IC * 4;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(awq_gemv_kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(awq_gemv_kernel, dim3((OC + 63) / 64), dim3(AWQ_THR), lds, stream, x, qw_rep, wscales, wzeros,
+                       bias, out, OC, IC, ncomp);
     return hipGetLastError();
 }
 

@@ -157,6 +157,22 @@ def test_awq_paths_bit_exact(qimg, oracle):
     np.testing.assert_array_equal(_bits(deq), want)
 
 
+@pytest.mark.parametrize("OC,IC,nc,bias", [(68, 64, 1, True), (60, 192, 6, False), (64, 576, 2, True),
+                                           (132, 640, 3, True), (72, 16384, 6, True)])
+def test_awq_gemv_edges_bit_exact(qimg, oracle, OC, IC, nc, bias):
+    """Channels past a workgroup's 64, one group, an odd number of groups (a
+    half-filled last stage), fewer stages than are in flight, the longest row."""
+    rng = np.random.default_rng(OC + IC)
+    rep = rng.integers(-2 ** 31, 2 ** 31, (IC // 8, OC), dtype=np.int64).astype(np.int32)
+    ws = oracle.bf16_bits_from_f32(rng.uniform(0.001, 0.02, (IC // 64, OC)).astype(np.float32))
+    wz = oracle.bf16_bits_from_f32(rng.uniform(-0.1, 0.1, (IC // 64, OC)).astype(np.float32))
+    b = oracle.bf16_bits_from_f32(rng.standard_normal(OC).astype(np.float32)) if bias else None
+    x = rng.standard_normal(IC).astype(np.float32)
+    out = qimg.linear_forward_awq(_f32(x), torch.from_numpy(rep).to(DEV), _bf16_bits_dev(ws), _bf16_bits_dev(wz), OC,
+                                  IC, bias=_bf16_bits_dev(b) if bias else None, num_components=nc)
+    np.testing.assert_array_equal(out.cpu().numpy()[0], oracle.awq_gemv(x, rep, ws, wz, OC, IC, 64, nc, bias_bits=b))
+
+
 @pytest.mark.parametrize("N,K,G", [(3072, 3072, 48), (128, 256, 2)])
 def test_nunchaku_conversions_bit_exact(qimg, oracle, N, K, G):
     rng = np.random.default_rng(N + G)
