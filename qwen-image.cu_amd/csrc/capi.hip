@@ -350,14 +350,13 @@ int qimg_sage_attention(const uint16_t* q_f16, const uint16_t* k_f16, const uint
     qimg::SageScratch ws;
     qimg::sage_scratch_layout(BH, S, D, scratch, &ws);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    st = hip_status(qimg::launch_sage_k_mean(k_f16, ws.k_mean, BH, S, D, s), fn);
-    if (st) return st;
-    st = hip_status(qimg::launch_sage_quant_q(q_f16, ws.q_i8, ws.q_scale, BH, S, D, s), fn);
+    st = hip_status(qimg::launch_sage_prep(q_f16, k_f16, v_f16, ws.q_i8, ws.q_scale, ws.k_mean, ws.v_t, BH, S, D, s),
+                    fn);
     if (st) return st;
     st = hip_status(qimg::launch_sage_quant_k(k_f16, ws.k_mean, ws.k_i8, ws.k_scale, BH, S, D, s), fn);
     if (st) return st;
-    return hip_status(qimg::launch_sage_attn(ws.q_i8, ws.k_i8, v_f16, ws.q_scale, ws.k_scale, out, out_dtype,
-                                             BH, S, D, sm_scale, causal, ws.v_t, s),
+    return hip_status(qimg::launch_sage_attn_vt(ws.q_i8, ws.k_i8, ws.v_t, ws.q_scale, ws.k_scale, out, out_dtype, BH,
+                                                S, D, sm_scale, causal, s),
                       fn);
 }
 

@@ -217,6 +217,10 @@ hipError_t launch_sage_quant_q(const uint16_t* q, int8_t* q_out, float* q_scale,
                                int D, hipStream_t stream);
 hipError_t launch_sage_quant_k(const uint16_t* k, const float* mean, int8_t* k_out,
                                float* k_scale, int BH, int S, int D, hipStream_t stream);
+// launch_sage_k_mean, launch_sage_quant_q and V's re-layout for
+// launch_sage_attn_vt in one launch (the same values).
+hipError_t launch_sage_prep(const uint16_t* q, const uint16_t* k, const uint16_t* v, int8_t* q_out, float* q_scale,
+                            float* mean, uint16_t* v_t, int BH, int S, int D, hipStream_t stream);
 hipError_t launch_sage_attn(const int8_t* q, const int8_t* k, const uint16_t* v,
                             const float* q_scale, const float* k_scale, void* out, int out_dtype,
                             int BH, int S, int D, float sm_scale, int causal, uint16_t* v_t,

@@ -60,18 +60,24 @@ __host__ __device__ constexpr int div_up(int a, int b) { return (a + b - 1) / b;
 // nothing), one fp32 add per token (the fp16 -> fp32 conversions stay off
 // the dependent chain), with the LDS reads of each group of 32 tokens
 // issued two groups ahead. Waves 1-3
-// stream KM_CHUNK-token chunks of k[h, :, d0:d0+32] (each lane 16 bytes =
+// stream chunks of k[h, :, d0:d0+32] (each lane 16 bytes =
 // 8 dims of 4 consecutive tokens), transpose 4 tokens x 8 dims in registers
 // and store them to LDS as [d][s] with 8-byte writes; rows are padded to a
 // pitch of 4 banks mod 64. Chunks are double-buffered in LDS,
 // and the loads run one chunk ahead of the LDS writes.
 constexpr int KM_DIMS = 32;                        // chains per workgroup
 constexpr int KM_G = KM_DIMS / 8;                  // 16-byte dim groups per token row
-constexpr int KM_CHUNK = 1024;                     // tokens per chunk
-constexpr int KM_PITCH = KM_CHUNK / 2 + 4;         // dwords per LDS row
+constexpr int KM_CHUNK = 1024;                     // tokens per chunk, the mean alone
 constexpr int KM_QPR = 64 / KM_G;                  // token quads per loader round
-constexpr int KM_ROUNDS = KM_CHUNK / 4 / KM_QPR;   // loader rounds per chunk
-constexpr int KM_MAXR = (KM_ROUNDS + 2) / 3;       // rounds per loader wave (at most)
+
+// Geometry of a mean with CHUNK tokens per LDS buffer.
+template <int CHUNK>
+struct KMean {
+    static constexpr int PITCH = CHUNK / 2 + 4;               // dwords per LDS row
+    static constexpr int ROUNDS = CHUNK / 4 / KM_QPR;         // loader rounds per chunk
+    static constexpr int MAXR = (ROUNDS + 2) / 3;             // rounds per loader wave (at most)
+    static constexpr int LDS_DWORDS = 2 * KM_DIMS * PITCH;
+};
 
 // acc + (fp16 token in the low / high half of v): the fp16 -> fp32
 // conversion is exact, so the sum is rounded once per token, as the
@@ -83,17 +89,22 @@ __device__ __forceinline__ float km_add_hi(float acc, uint32_t v) {
     return acc + f16_to_f32(static_cast<uint16_t>(v >> 16));
 }
 
-__global__ __launch_bounds__(256) void k_mean_kernel(const uint16_t* __restrict__ k, float* __restrict__ mean,
-                                                     int S, int D) {
-    __shared__ __attribute__((aligned(16))) uint32_t tile[2][KM_DIMS * KM_PITCH];
+// Mean of slice `unit` (head unit / (D / 32), dims 32 (unit % (D / 32)) ..)
+// by a workgroup of 256 threads; tile holds KMean<CHUNK>::LDS_DWORDS.
+template <int CHUNK>
+__device__ __forceinline__ void k_mean_slice(const uint16_t* __restrict__ k, float* __restrict__ mean, int S, int D,
+                                             int unit, uint32_t* tile) {
+    constexpr int PITCH = KMean<CHUNK>::PITCH;
+    constexpr int ROUNDS = KMean<CHUNK>::ROUNDS;
+    constexpr int MAXR = KMean<CHUNK>::MAXR;
     const int slices = D / KM_DIMS;
-    const int h = blockIdx.x / slices;
-    const int d0 = (blockIdx.x % slices) * KM_DIMS;
+    const int h = unit / slices;
+    const int d0 = (unit % slices) * KM_DIMS;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const uint16_t* src = k + static_cast<int64_t>(h) * S * D + d0;
-    const int nchunk = div_up(S, KM_CHUNK);
+    const int nchunk = div_up(S, CHUNK);
 
     // loader lane: dim group g = lane % KM_G, token quad KM_QPR * round +
     // lane / KM_G. issue() starts the loads of a chunk into registers,
@@ -102,25 +113,25 @@ __global__ __launch_bounds__(256) void k_mean_kernel(const uint16_t* __restrict_
     // whole chunk of the sum. (A second register set, two chunks in flight,
     // measured slower: the compiler's in-order vmcnt waits drain both.)
     const int g = lane % KM_G;
-    u32x4 v[1][KM_MAXR][4];
+    u32x4 v[1][MAXR][4];
     auto issue = [&](int c, int set) {
 #pragma unroll
-        for (int r = 0; r < KM_MAXR; ++r) {
+        for (int r = 0; r < MAXR; ++r) {
             const int round = (wave - 1) + 3 * r;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int s = c * KM_CHUNK + 4 * (KM_QPR * round + lane / KM_G) + i;
+                const int s = c * CHUNK + 4 * (KM_QPR * round + lane / KM_G) + i;
                 v[set][r][i] = (u32x4){0u, 0u, 0u, 0u};
-                if (round < KM_ROUNDS && s < S)
+                if (round < ROUNDS && s < S)
                     v[set][r][i] = *reinterpret_cast<const u32x4*>(src + static_cast<int64_t>(s) * D + 8 * g);
             }
         }
     };
     auto commit = [&](int buf, int set) {
 #pragma unroll
-        for (int r = 0; r < KM_MAXR; ++r) {
+        for (int r = 0; r < MAXR; ++r) {
             const int round = (wave - 1) + 3 * r;
-            if (round >= KM_ROUNDS) continue;
+            if (round >= ROUNDS) continue;
             const int tq = KM_QPR * round + lane / KM_G;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -130,7 +141,7 @@ __global__ __launch_bounds__(256) void k_mean_kernel(const uint16_t* __restrict_
                 const uint32_t t0 = (v[set][r][0][w] >> sh) & 0xffffu, t1 = (v[set][r][1][w] >> sh) & 0xffffu;
                 const uint32_t t2 = (v[set][r][2][w] >> sh) & 0xffffu, t3 = (v[set][r][3][w] >> sh) & 0xffffu;
                 const int d = 8 * g + e;
-                uint32_t* dst = &tile[buf][d * KM_PITCH + 2 * tq];
+                uint32_t* dst = &tile[(buf * KM_DIMS + d) * PITCH + 2 * tq];
                 *reinterpret_cast<uint2*>(dst) = make_uint2(t0 | (t1 << 16), t2 | (t3 << 16));
             }
         }
@@ -151,8 +162,8 @@ __global__ __launch_bounds__(256) void k_mean_kernel(const uint16_t* __restrict_
                 if (c + 2 < nchunk) issue(c + 2, 0);
             }
         } else {
-            const int n = min(KM_CHUNK, S - c * KM_CHUNK);
-            const uint32_t* row = &tile[buf][(lane % KM_DIMS) * KM_PITCH];
+            const int n = min(CHUNK, S - c * CHUNK);
+            const uint32_t* row = &tile[(buf * KM_DIMS + lane % KM_DIMS) * PITCH];
             auto rd = [&](int t8) { return *reinterpret_cast<const u32x4*>(row + 4 * t8); };
             // groups of 32 tokens, read two groups ahead in two register
             // sets; a read past the chunk's last full group re-reads group
@@ -192,18 +203,20 @@ __global__ __launch_bounds__(256) void k_mean_kernel(const uint16_t* __restrict_
     if (tid < KM_DIMS) mean[static_cast<int64_t>(h) * D + d0 + tid] = sum / fmaxf(static_cast<float>(S), 1.0f);
 }
 
+__global__ __launch_bounds__(256) void k_mean_kernel(const uint16_t* __restrict__ k, float* __restrict__ mean,
+                                                     int S, int D) {
+    __shared__ __attribute__((aligned(16))) uint32_t tile[KMean<KM_CHUNK>::LDS_DWORDS];
+    k_mean_slice<KM_CHUNK>(k, mean, S, D, blockIdx.x, tile);
+}
+
 // ---------------------------------------------------------------- Q quant
 // Block = 256 threads for one (head, 128-token block). Thread t holds token
 // t/2, half t%2 of the head dim (D/2 values).
 template <int D>
-__global__ __launch_bounds__(256) void quant_q_kernel(const uint16_t* __restrict__ q,
-                                                      int8_t* __restrict__ q_out,
-                                                      float* __restrict__ q_scale, int S) {
+__device__ __forceinline__ void quant_q_block(const uint16_t* __restrict__ q, int8_t* __restrict__ q_out,
+                                              float* __restrict__ q_scale, int S, int b, int h, float (*red)[2],
+                                              float* inv_s) {
     constexpr int HD = D / 2;
-    __shared__ float red[QBLK][2];
-    __shared__ float inv_s[32];
-    const int b = blockIdx.x;
-    const int h = blockIdx.y;
     const int tid = threadIdx.x;
     const int tok = b * QBLK + (tid >> 1);
     const int part = tid & 1;
@@ -256,6 +269,15 @@ __global__ __launch_bounds__(256) void quant_q_kernel(const uint16_t* __restrict
         }
         reinterpret_cast<u32x4*>(dst)[c] = pk;
     }
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void quant_q_kernel(const uint16_t* __restrict__ q,
+                                                      int8_t* __restrict__ q_out,
+                                                      float* __restrict__ q_scale, int S) {
+    __shared__ float red[QBLK][2];
+    __shared__ float inv_s[32];
+    quant_q_block<D>(q, q_out, q_scale, S, blockIdx.x, blockIdx.y, red, inv_s);
 }
 
 // ---------------------------------------------------------------- K quant
@@ -392,11 +414,8 @@ __device__ __forceinline__ int vt_key_of_pos(int p) {
 }
 
 template <int D>
-__global__ __launch_bounds__(256) void v_relayout_kernel(const uint16_t* __restrict__ v,
-                                                         uint16_t* __restrict__ vt, int S) {
-    __shared__ uint16_t tile[KTILE][D + 2];
-    const int kt = blockIdx.x;
-    const int h = blockIdx.y;
+__device__ __forceinline__ void v_relayout_tile(const uint16_t* __restrict__ v, uint16_t* __restrict__ vt, int S,
+                                                int kt, int h, uint16_t (*tile)[D + 2]) {
     const int tid = threadIdx.x;
     const uint16_t* src = v + static_cast<int64_t>(h) * S * D;
     // load 64 x D, 16 bytes per piece
@@ -427,6 +446,51 @@ __global__ __launch_bounds__(256) void v_relayout_kernel(const uint16_t* __restr
         }
         reinterpret_cast<u32x4*>(dst + d * KTILE)[c] = o;
     }
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void v_relayout_kernel(const uint16_t* __restrict__ v,
+                                                         uint16_t* __restrict__ vt, int S) {
+    __shared__ uint16_t tile[KTILE][D + 2];
+    v_relayout_tile<D>(v, vt, S, blockIdx.x, blockIdx.y, tile);
+}
+
+// ------------------------------------------------ K mean, Q quant, V re-layout
+// The three passes of an attention call that do not depend on each other in
+// one launch: workgroups [0, n_mean) take the K mean's slices, the next
+// n_q the Q quantization's (head, 128-token) blocks, the rest V's
+// (head, 64-key) tiles. BH * D / 32 workgroups of latency-bound dependent
+// adds leave most CUs idle, and the two HBM-bound passes run there.
+// The whole attention call, against the passes one after another: 24 x 4352
+// x 128 273.3 -> 252.7 us (mean 27 + Q 12 + V 9.6 before), 24 x 1301 64.6 ->
+// 55.2 us. The mean's chunk is 512 tokens (66 KB of LDS) instead of 1024
+// (132 KB), so that two workgroups share a CU and its first chunk arrives
+// sooner; 256 measured 254.7 and 55.0 us.
+constexpr int PREP_CHUNK = 512;
+template <int D>
+__global__ __launch_bounds__(256) void sage_prep_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                                                        const uint16_t* __restrict__ v, int8_t* __restrict__ q_out,
+                                                        float* __restrict__ q_scale, float* __restrict__ mean,
+                                                        uint16_t* __restrict__ vt, int S, int n_mean, int n_q) {
+    constexpr int LDS_BYTES = KMean<PREP_CHUNK>::LDS_DWORDS * 4;
+    static_assert(LDS_BYTES >= KTILE * (D + 2) * 2 && LDS_BYTES >= (2 * QBLK + 32) * 4, "one buffer for every pass");
+    __shared__ __attribute__((aligned(16))) uint32_t lds[LDS_BYTES / 4];
+    int unit = blockIdx.x;
+    if (unit < n_mean) {
+        k_mean_slice<PREP_CHUNK>(k, mean, S, D, unit, lds);
+        return;
+    }
+    unit -= n_mean;
+    if (unit < n_q) {
+        const int per_head = div_up(S, QBLK);
+        float(*red)[2] = reinterpret_cast<float(*)[2]>(lds);
+        quant_q_block<D>(q, q_out, q_scale, S, unit % per_head, unit / per_head, red,
+                         reinterpret_cast<float*>(lds) + 2 * QBLK);
+        return;
+    }
+    unit -= n_q;
+    const int per_head = div_up(S, KTILE);
+    v_relayout_tile<D>(v, vt, S, unit % per_head, unit / per_head, reinterpret_cast<uint16_t(*)[D + 2]>(lds));
 }
 
 // Zeros at the positions of keys S .. 64 ceil(S/64) - 1 of the last key
@@ -1076,6 +1140,37 @@ hipError_t launch_sage_quant_q(const uint16_t* q, int8_t* q_out, float* q_scale,
     return hipGetLastError();
 }
 
+static hipError_t launch_v_relayout(const uint16_t* v, uint16_t* v_t, int BH, int S, int D, hipStream_t stream) {
+    dim3 grid(div_up(S, KTILE), BH);
+    if (D == 128)
+        hipLaunchKernelGGL(v_relayout_kernel<128>, grid, dim3(256), 0, stream, v, v_t, S);
+    else
+        hipLaunchKernelGGL(v_relayout_kernel<64>, grid, dim3(256), 0, stream, v, v_t, S);
+    return hipGetLastError();
+}
+
+hipError_t launch_sage_prep(const uint16_t* q, const uint16_t* k, const uint16_t* v, int8_t* q_out, float* q_scale,
+                            float* mean, uint16_t* v_t, int BH, int S, int D, hipStream_t stream) {
+    const int64_t n_mean = static_cast<int64_t>(BH) * (D / KM_DIMS);
+    const int64_t n_q = static_cast<int64_t>(BH) * div_up(S, QBLK);
+    const int64_t n_v = static_cast<int64_t>(BH) * div_up(S, KTILE);
+    // a launch holds fewer than 2^32 threads; millions of heads of a few
+    // tokens take the passes one by one
+    if ((n_mean + n_q + n_v) * 256 >= int64_t{1} << 32) {
+        hipError_t e = launch_sage_k_mean(k, mean, BH, S, D, stream);
+        if (e == hipSuccess) e = launch_sage_quant_q(q, q_out, q_scale, BH, S, D, stream);
+        return e == hipSuccess ? launch_v_relayout(v, v_t, BH, S, D, stream) : e;
+    }
+    const dim3 grid(static_cast<unsigned>(n_mean + n_q + n_v));
+    if (D == 128)
+        hipLaunchKernelGGL(sage_prep_kernel<128>, grid, dim3(256), 0, stream, q, k, v, q_out, q_scale, mean, v_t, S,
+                           static_cast<int>(n_mean), static_cast<int>(n_q));
+    else
+        hipLaunchKernelGGL(sage_prep_kernel<64>, grid, dim3(256), 0, stream, q, k, v, q_out, q_scale, mean, v_t, S,
+                           static_cast<int>(n_mean), static_cast<int>(n_q));
+    return hipGetLastError();
+}
+
 hipError_t launch_sage_quant_k(const uint16_t* k, const float* mean, int8_t* k_out,
                                float* k_scale, int BH, int S, int D, hipStream_t stream) {
     dim3 grid(div_up(S, KTILE), BH);
@@ -1118,12 +1213,7 @@ hipError_t launch_sage_attn(const int8_t* q, const int8_t* k, const uint16_t* v,
                             const float* q_scale, const float* k_scale, void* out, int out_dtype,
                             int BH, int S, int D, float sm_scale, int causal, uint16_t* v_t,
                             hipStream_t stream) {
-    dim3 vgrid(div_up(S, KTILE), BH);
-    if (D == 128)
-        hipLaunchKernelGGL(v_relayout_kernel<128>, vgrid, dim3(256), 0, stream, v, v_t, S);
-    else
-        hipLaunchKernelGGL(v_relayout_kernel<64>, vgrid, dim3(256), 0, stream, v, v_t, S);
-    hipError_t e = hipGetLastError();
+    const hipError_t e = launch_v_relayout(v, v_t, BH, S, D, stream);
     if (e != hipSuccess) return e;
     return launch_sage_attn_vt(q, k, v_t, q_scale, k_scale, out, out_dtype, BH, S, D, sm_scale, causal, stream);
 }

@@ -211,3 +211,18 @@ def test_sage_joint_attention_c3_inputs(qimg, oracle):
     exact = np.matmul(p64 / p64.sum(-1, keepdims=True), v.astype(np.float64))
     rel, cos = _metrics(got[:, r0:r0 + 128], exact)
     assert rel <= 2e-2 and cos >= 0.999, (rel, cos)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("BH,S", [(1, 1), (5, 31), (2, 77), (3, 511), (2, 512), (1, 513), (7, 1055), (24, 1301)])
+def test_sage_call_equals_its_passes(qimg, BH, S, D):
+    """The call's one launch of K mean, Q quantization and V re-layout gives
+    the values of the separate passes, around the mean's 512-token chunks
+    and the 128- and 64-token blocks."""
+    q, k, v = (_dev(a) for a in _inputs(BH, S, D, 3 * S + D))
+    got = qimg.attention_forward_sage_fp16io(q, k, v, 1.0 / math.sqrt(D))
+    qi, qs = qimg.sage_quant_q(q)
+    ki, ks = qimg.sage_quant_k(k, qimg.sage_k_mean(k))
+    ref = qimg.sage_attn_quantized(qi, ki, v, qs, ks, 1.0 / math.sqrt(D))
+    torch.cuda.synchronize()
+    assert torch.equal(got, ref.to(got.dtype))
