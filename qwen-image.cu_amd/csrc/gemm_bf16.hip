@@ -15,16 +15,18 @@
 // Shapes (M = tokens): img_in 3072 x 64, txt_in 3072 x 3584, norm_out
 // 6144 x 3072 at M = 1 (or 2), proj_out 64 x 3072. They are bound by reading
 // the weights (norm_out, txt_in) or the activations (proj_out) or by writing
-// the output (img_in), so the kernel is built like the small-M quantized
-// linear: a workgroup owns a 32x32 or 64x64 output tile, its four waves
-// split K in 32-element blocks dealt round-robin (every operand byte is
-// read by one wave), and the partial tiles are summed through LDS in wave
-// order. Operands go straight from global memory into MFMA fragment
-// registers with buffer loads (rows past M or N and blocks past K read as
-// zero), DEPTH blocks in flight per wave. v_mfma_f32_32x32x16_bf16: lane
-// (row r = lane%32, half h = lane/32) of a 32-row block holds, for k-step s
-// of K block kb, the 8 elements kb*32 + 16h + 8s .. +7; both operands use
-// the same assignment, so each dot product covers every k once.
+// the output (img_in). Short K (img_in) takes gemm_bf16_shortk_kernel, K of
+// whole 128-element stages gemm_bf16_dma_kernel, other multiples of 32
+// gemm_bf16_kernel, built like the small-M quantized linear: a workgroup owns
+// a 32x32 or 64x64 output tile, its four waves split K in 32-element blocks
+// dealt round-robin (every operand byte is read by one wave), and the partial
+// tiles are summed through LDS in wave order. Operands go straight from global
+// memory into MFMA fragment registers with buffer loads (rows past M or N and
+// blocks past K read as zero), DEPTH blocks in flight per wave.
+// v_mfma_f32_32x32x16_bf16: lane (row r = lane%32, half h = lane/32) of a
+// 32-row block holds, for k-step s of K block kb, the 8 elements
+// kb*32 + 16h + 8s .. +7; both operands use the same assignment, so each dot
+// product covers every k once.
 #include <utility>
 
 #include "qimg_device.h"
@@ -36,6 +38,8 @@ namespace {
 
 constexpr int BF_THR = 256;  // four waves, one K quarter each
 constexpr int BF_KB = 32;    // elements of K per block
+constexpr int SK_M = 64, SK_N = 128;  // tile of the short-K kernel
+constexpr int kShortKMaxN = 1 << 22;  // its tile's output rows stay below 2^31 bytes (kOob out of range)
 constexpr int kRsrcWord3 = 0x00020000;  // raw unswizzled buffer (gfx9 family)
 constexpr uint32_t kOob = 0x80000000u;  // offset >= num_records: reads zero
 
@@ -248,92 +252,335 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_kernel(const void* __restric
     }
 }
 
-// Short K (img_in: K = 64): the four waves of a workgroup own the four
-// 32x32 blocks of a 64x64 tile and each runs the whole of K, so no partial
-// tiles are reduced and no LDS is used; the operand loads and the fragment
-// layout are those of gemm_bf16_kernel, the products are summed in K-block
-// order, and each lane stores its 16 outputs (row m = lane%32, columns
-// 8g + 4(lane/32) + c) as four 16-byte runs.
+// Short K (img_in: K = 64): bound by writing the output. A workgroup owns 64
+// rows x 128 columns, each wave 64 x 32 (two 32x32 blocks), and runs the
+// whole of K, so no partial tiles are reduced; the operand loads and fragments
+// are those of gemm_bf16_kernel with x as the A operand, two K blocks loaded
+// at a time, the products summed in K-block order. Each block of 32 rows then
+// goes through LDS, so that a store instruction writes 512 contiguous bytes of
+// two rows. Tiles are numbered n first, so that workgroups in flight together
+// write whole output rows. 4096x3072x64: 29.9 us with 16-byte stores of 32
+// rows per instruction, 23.8 with 128-byte lines of two rows straight from
+// the accumulators, 21.6 as it is (50 MB: 2.3 TB/s).
 template <bool XF32, bool GELU>
 __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __restrict__ X,
                                                                   const uint16_t* __restrict__ Wt,
                                                                   const uint16_t* __restrict__ bias,
                                                                   float* out, int M, int N, int K, int accumulate) {
     constexpr int XE = XF32 ? 4 : 2;
-    const int tiles_m = (M + 63) / 64;
-    const int tiles_n = (N + 63) / 64;
+    constexpr int PITCH = SK_N + 4;
+    __shared__ __attribute__((aligned(16))) float stage[32 * PITCH];
+    const int tiles_m = (M + SK_M - 1) / SK_M;
+    const int tiles_n = (N + SK_N - 1) / SK_N;
     const int logical = xcd_remap(blockIdx.x, tiles_m * tiles_n);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = (logical % tiles_m) * 64 + 32 * (wave >> 1);
-    const int n0 = (logical / tiles_m) * 64 + 32 * (wave & 1);
+    const int m0 = (logical / tiles_n) * SK_M;
+    const int n0 = (logical % tiles_n) * SK_N;
     const int r = lane & 31;
     const int h = lane >> 5;
+    const int n = n0 + 32 * wave + r;
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void*>(X), 0, static_cast<int>(static_cast<int64_t>(M) * K * XE), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(Wt), 0, static_cast<int>(static_cast<int64_t>(N) * K * 2), kRsrcWord3);
-    const uint32_t ox = (static_cast<uint32_t>(m0 + r) * K + 16 * h) * XE | (m0 + r < M ? 0u : kOob);
-    const uint32_t ow = (static_cast<uint32_t>(n0 + r) * K + 16 * h) * 2 | (n0 + r < N ? 0u : kOob);
-    float bv[16];
+    const __amdgpu_buffer_rsrc_t rb =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(bias), 0, bias != nullptr ? N * 2 : 0, kRsrcWord3);
+    // the tile's rows of out, those past M out of range
+    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+        out + static_cast<int64_t>(m0) * N, 0, (M - m0 < SK_M ? M - m0 : SK_M) * N * 4, kRsrcWord3);
+    uint32_t ox[2];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int n = n0 + 8 * (e >> 2) + 4 * h + (e & 3);
-        bv[e] = bias != nullptr ? bf16_to_f32(bias[n < N ? n : N - 1]) : 0.0f;
-    }
-    v16f acc;
+    for (int i = 0; i < 2; ++i)
+        ox[i] = m0 + 32 * i + r < M ? (static_cast<uint32_t>(m0 + 32 * i + r) * K + 16 * h) * XE : kOob;
+    const uint32_t ow = n < N ? (static_cast<uint32_t>(n) * K + 16 * h) * 2 : kOob;
+    v16f acc[2];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
     const int nkb = K / BF_KB;
-    for (int kb = 0; kb < nkb; ++kb) {
-        const uint32_t dx = static_cast<uint32_t>(kb) * BF_KB * XE;
-        const uint32_t dw = static_cast<uint32_t>(kb) * BF_KB * 2;
-        v8bf fx[2], fw[2];
-        if constexpr (XF32) {
-            v4f xv[4];
+    for (int k2 = 0; k2 < nkb; k2 += 2) {
+        v4i xr[2][2][XF32 ? 4 : 2], wr[2][2];
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
-                xv[s] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rx, ((ox + dx) | (ox & kOob)) + 16 * s, 0, 0));
-            f32x16_to_frags(xv, fx[0], fx[1]);
-        } else {
+        for (int d = 0; d < 2; ++d) {
+            const uint32_t bad = k2 + d < nkb ? 0u : kOob;  // past K: zeros
+            const uint32_t kb = static_cast<uint32_t>(k2 + d) * BF_KB;
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
-                fx[s] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(rx, ((ox + dx) | (ox & kOob)) + 16 * s, 0, 0));
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q = 0; q < (XF32 ? 4 : 2); ++q)
+                    xr[d][i][q] = __builtin_bit_cast(
+                        v4i, __builtin_amdgcn_raw_buffer_load_b128(rx, ((ox[i] + kb * XE + 16 * q) | (ox[i] & kOob) | bad), 0, 0));
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                wr[d][q] = __builtin_bit_cast(
+                    v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, ((ow + kb * 2 + 16 * q) | (ow & kOob) | bad), 0, 0));
         }
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
-            fw[s] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(rw, ((ow + dw) | (ow & kOob)) + 16 * s, 0, 0));
+        for (int d = 0; d < 2; ++d) {
+            v8bf fx[2][2];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[s], fx[s], acc, 0, 0, 0);
+            for (int i = 0; i < 2; ++i) {
+                if constexpr (XF32) {
+                    v4f xv[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) xv[q] = __builtin_bit_cast(v4f, xr[d][i][q]);
+                    f32x16_to_frags(xv, fx[i][0], fx[i][1]);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) fx[i][q] = __builtin_bit_cast(v8bf, xr[d][i][q]);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[i][q], __builtin_bit_cast(v8bf, wr[d][q]),
+                                                                     acc[i], 0, 0, 0);
+        }
     }
-    const int m = m0 + r;
-    if (m >= M) return;
+    const float bv = bf16_to_f32(
+        static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(rb, static_cast<uint32_t>(n) * 2, 0, 0)));
+    const bool vec_ok = (N & 3) == 0;
+    const int sc = 4 * (threadIdx.x & 31);  // columns this thread stores
+    const int sr = threadIdx.x >> 5;        // and its first row
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const int nb = n0 + 8 * g + 4 * h;
-        if (nb >= N) continue;
-        float* o = out + static_cast<int64_t>(m) * N + nb;
-        float prev[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < 2; ++i) {
+        // element e: row 32 i + 8 (e / 4) + 4 h + e % 4, column n
+        float v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = acc[i][e];
         if (accumulate) {
+            float prev[16];
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (nb + c < N) prev[c] = o[c];
+            for (int e = 0; e < 16; ++e)
+                prev[e] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(
+                               ro, n < N ? (static_cast<uint32_t>(32 * i + 8 * (e >> 2) + 4 * h + (e & 3)) * N + n) * 4 : kOob, 0, 0));
+#pragma unroll
+            for (int e = 0; e < 16; ++e) v[e] = v[e] + prev[e];
+        }
+        if (i > 0) __syncthreads();  // the first block's stores have read the stage
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            if (bias != nullptr) v[e] = v[e] + bv;
+            if (GELU) v[e] = gelu_tanh(v[e]);
+            stage[(8 * (e >> 2) + 4 * h + (e & 3)) * PITCH + 32 * wave + r] = v[e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int row = sr + 8 * q;
+            const v4f t = *reinterpret_cast<const v4f*>(stage + row * PITCH + sc);
+            const uint32_t o = (static_cast<uint32_t>(32 * i + row) * N + n0 + sc) * 4;
+            if (vec_ok) {
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, t), ro, n0 + sc < N ? o : kOob, 0, 0);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float tc = t[c];
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(tc), ro, n0 + sc + c < N ? o + 4 * c : kOob,
+                                                          0, 0);
+                }
+            }
+        }
+    }
+}
+
+// Long K (txt_in, norm_out, proj_out, the INT4 linears' down factor): tiles
+// of TM rows x TN columns whose operands stream through LDS. A stage is 128
+// elements of K of the tile's x and w rows, filled by direct global->LDS DMA
+// of whole lines (1 KB per instruction; the direct fragment loads of
+// gemm_bf16_kernel touch 16 to 64 bytes of each of 32 lines) into a ring of
+// NS stages, NS - 1 in flight. The four waves take 32 elements of K each and
+// compute the whole tile (v_mfma_f32_16x16x32_bf16, w as the A operand), so
+// each operand byte leaves LDS once; x is rounded to bf16 on the fragments.
+// The partial tiles are summed through LDS in wave order, and the stores run
+// along n. One barrier per stage: stage s has landed in every wave, and every
+// wave is done with stage s - 1, whose slot is refilled right after.
+// LDS chunk c of row r sits at c ^ (r & 15): the 16 rows of a fragment read
+// fall on 16 different bank groups.
+// Rows past M and N re-read the last row and are not stored.
+// Measured against gemm_bf16_kernel (us, fp32 x): txt_in 256x3072x3584 48 ->
+// 24, proj_out 4096x64x3072 25 -> 11 (50 MB of x: 4.6 TB/s), norm_out
+// 1x6144x3072 11 -> 7.9 (38 MB of w: 4.8 TB/s); the INT4 down factor
+// 4096x32x3072 (bf16 x) 15.7 -> 6.7. txt_in is bound by the 1.4 MB each of
+// its 192 workgroups reads through its CU's port with 96 KB in flight.
+template <bool XF32, int TM, int TN>
+struct BfDma {
+    static constexpr int KS = 128;                        // K elements per stage
+    static constexpr int XE = XF32 ? 4 : 2;
+    static constexpr int XROW = KS * XE, WROW = KS * 2;   // bytes per row of a stage
+    static constexpr int XB = TM * XROW, WB = TN * WROW;
+    static constexpr int STAGE = XB + WB;
+    static constexpr int NS = 144 * 1024 / STAGE < 8 ? 144 * 1024 / STAGE : 8;
+    static constexpr int XI = XB / 4096, WI = WB / 4096;  // DMA instructions per wave and stage
+    static constexpr int PER = XI + WI;
+    static_assert(XB % 4096 == 0 && WB % 4096 == 0 && NS >= 3 && (NS - 1) * PER <= 63, "stage split over four waves");
+    static_assert(NS * STAGE >= 4 * TM * (TN + 4) * 4, "the partial tiles reuse the ring");
+};
+
+template <bool XF32, int TM, int TN, bool GELU>
+__global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __restrict__ X,
+                                                               const uint16_t* __restrict__ Wt,
+                                                               const uint16_t* __restrict__ bias, float* out, int M,
+                                                               int N, int K, int accumulate) {
+    using G = BfDma<XF32, TM, TN>;
+    constexpr int NS = G::NS, PER = G::PER, XI = G::XI;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * G::STAGE];
+
+    const int tiles_m = (M + TM - 1) / TM;
+    const int tiles_n = (N + TN - 1) / TN;
+    const int logical = xcd_remap(blockIdx.x, tiles_m * tiles_n);
+    // tiles that share rows of the larger operand are numbered in a row: one
+    // XCD's L2 reads them once (proj_out's x, txt_in's w)
+    const bool x_larger = static_cast<int64_t>(M) * G::XE > static_cast<int64_t>(N) * 2;
+    const int m0 = (x_larger ? logical / tiles_n : logical % tiles_m) * TM;
+    const int n0 = (x_larger ? logical % tiles_n : logical / tiles_m) * TN;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    // bias of the four columns this thread stores in every row it stores
+    const int col = n0 + 4 * (static_cast<int>(threadIdx.x) % (TN / 4));
+    float bv[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) bv[c] = bias != nullptr ? bf16_to_f32(bias[col + c < N ? col + c : N - 1]) : 0.0f;
+
+    // DMA instruction j of this wave fills KB 4 j + wave of the stage (x
+    // rows, then w rows)
+    const uint8_t* src[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const bool is_x = j < XI;
+        const int rb = is_x ? G::XROW : G::WROW;  // bytes per row
+        const int off = (4 * (is_x ? j : j - XI) + wave) * 1024 + lane * 16;
+        const int row = off / rb;
+        const int c = ((off % rb) >> 4) ^ (row & 15);
+        if (is_x) {
+            const int gm = m0 + row < M ? m0 + row : M - 1;
+            src[j] = static_cast<const uint8_t*>(X) + static_cast<int64_t>(gm) * K * G::XE + c * 16;
+        } else {
+            const int gn = n0 + row < N ? n0 + row : N - 1;
+            src[j] = reinterpret_cast<const uint8_t*>(Wt) + static_cast<int64_t>(gn) * K * 2 + c * 16;
+        }
+    }
+    auto issue = [&](int s, int slot) {
+        uint8_t* dst = lds + slot * G::STAGE + wave * 1024;
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src[j] + static_cast<int64_t>(s) * (j < XI ? G::XROW : G::WROW)),
+                                             (lds_ptr_t)(dst + j * 4096), 16, 0, 1);
+    };
+
+    const int r = lane & 15;
+    const int kq = lane >> 4;
+    v4f acc[TM / 16][TN / 16];
+#pragma unroll
+    for (int i = 0; i < TM / 16; ++i)
+#pragma unroll
+        for (int j = 0; j < TN / 16; ++j) acc[i][j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    // lane (row r, kq) of a fragment holds elements 32 wave + 8 kq .. +7
+    auto compute = [&](int slot) {
+        const uint8_t* xs = lds + slot * G::STAGE;
+        const uint8_t* ws = xs + G::XB;
+        v8bf fx[TM / 16], fw[TN / 16];
+#pragma unroll
+        for (int j = 0; j < TN / 16; ++j)
+            fw[j] = *reinterpret_cast<const v8bf*>(ws + (16 * j + r) * G::WROW + (((4 * wave + kq) ^ r) << 4));
+#pragma unroll
+        for (int i = 0; i < TM / 16; ++i) {
+            const uint8_t* row = xs + (16 * i + r) * G::XROW;
+            if constexpr (XF32) {
+                const v4f lo = *reinterpret_cast<const v4f*>(row + (((8 * wave + 2 * kq) ^ r) << 4));
+                const v4f hi = *reinterpret_cast<const v4f*>(row + (((8 * wave + 2 * kq + 1) ^ r) << 4));
+                fx[i] = __builtin_bit_cast(v8bf, (v4i){static_cast<int>(pack_bf16x2(lo[0], lo[1])),
+                                                       static_cast<int>(pack_bf16x2(lo[2], lo[3])),
+                                                       static_cast<int>(pack_bf16x2(hi[0], hi[1])),
+                                                       static_cast<int>(pack_bf16x2(hi[2], hi[3]))});
+            } else {
+                fx[i] = *reinterpret_cast<const v8bf*>(row + (((4 * wave + kq) ^ r) << 4));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TM / 16; ++i)
+#pragma unroll
+            for (int j = 0; j < TN / 16; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[j], fx[i], acc[i][j], 0, 0, 0);
+    };
+
+    const int T = K / G::KS;
+#pragma unroll
+    for (int d = 0; d < NS - 1; ++d)
+        if (d < T) issue(d, d);
+    int s = 0, slot = 0;
+    for (; s + NS - 1 < T; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<(NS - 2) * PER>();
+        wait_lgkmcnt0();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        issue(s + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+        compute(slot);
+        slot = slot + 1 == NS ? 0 : slot + 1;
+    }
+    // the last NS - 1 stages: nothing left to refill
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<0>();
+    wait_lgkmcnt0();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    for (; s < T; ++s) {
+        compute(slot);
+        slot = slot + 1 == NS ? 0 : slot + 1;
+    }
+    __syncthreads();  // every wave is done with the ring: the partial tiles take its place
+
+    constexpr int PITCH = TN + 4;
+    float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int i = 0; i < TM / 16; ++i)
+#pragma unroll
+        for (int j = 0; j < TN / 16; ++j)
+            *reinterpret_cast<v4f*>(red + (wave * TM + 16 * i + r) * PITCH + 16 * j + 4 * kq) = acc[i][j];
+    __syncthreads();
+    const bool vec_ok = (N & 3) == 0;
+#pragma unroll
+    for (int q = 0; q < (TM * TN / 4 + BF_THR - 1) / BF_THR; ++q) {
+        const int idx = static_cast<int>(threadIdx.x) + BF_THR * q;
+        const int row = idx / (TN / 4);
+        const int m = m0 + row;
+        if (row >= TM || m >= M || col >= N) continue;
+        const float* p = red + row * PITCH + (col - n0);
+        v4f sum = *reinterpret_cast<const v4f*>(p);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const v4f*>(p + w * TM * PITCH);
+        float* o = out + static_cast<int64_t>(m) * N + col;
+        v4f prev = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (accumulate) {
+            if (vec_ok) {
+                prev = *reinterpret_cast<const v4f*>(o);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (col + c < N) prev[c] = o[c];
+            }
         }
         float v[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            float t = acc[4 * g + c];
+            float t = sum[c];
             if (accumulate) t = t + prev[c];
-            if (bias != nullptr) t = t + bv[4 * g + c];
+            if (bias != nullptr) t = t + bv[c];
             if (GELU) t = gelu_tanh(t);
             v[c] = t;
         }
-        if ((N & 3) == 0) {
+        if (vec_ok) {
             *reinterpret_cast<v4f*>(o) = (v4f){v[0], v[1], v[2], v[3]};
         } else {
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                if (nb + c < N) o[c] = v[c];
+                if (col + c < N) o[c] = v[c];
         }
     }
 }
@@ -381,6 +628,46 @@ hipError_t launch_tiled_bf16(const void* x, int M, int K, const uint16_t* w, int
     return hipGetLastError();
 }
 
+template <bool XF32, int TM, int TN>
+hipError_t launch_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N, const uint16_t* bias, float* out,
+                           int gelu, int accumulate, hipStream_t stream) {
+    const int tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN);
+    if (gelu)
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, true>), dim3(tiles), dim3(BF_THR), 0, stream, x, w,
+                           bias, out, M, N, K, accumulate);
+    else
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, false>), dim3(tiles), dim3(BF_THR), 0, stream, x, w,
+                           bias, out, M, N, K, accumulate);
+    return hipGetLastError();
+}
+
+// The tile of gemm_bf16_dma_kernel: one workgroup per CU streams its rows
+// through the CU's L2 port, so the launch takes about the rounds of 256
+// workgroups times the bytes of a tile's rows.
+template <bool XF32>
+hipError_t launch_best_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N, const uint16_t* bias,
+                                float* out, int gelu, int accumulate, hipStream_t stream) {
+    constexpr int tm[] = {64, 64, 32, 32, 16, 16}, tn[] = {64, 32, 64, 32, 64, 32};
+    int best = 0;
+    int64_t best_cost = INT64_MAX;
+    for (int i = 0; i < 6; ++i) {
+        const int64_t tiles = static_cast<int64_t>((M + tm[i] - 1) / tm[i]) * ((N + tn[i] - 1) / tn[i]);
+        const int64_t cost = (tiles + 255) / 256 * (tm[i] * (XF32 ? 4 : 2) + tn[i] * 2);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = i;
+        }
+    }
+    switch (best) {
+    case 0: return launch_dma_bf16<XF32, 64, 64>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+    case 1: return launch_dma_bf16<XF32, 64, 32>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+    case 2: return launch_dma_bf16<XF32, 32, 64>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+    case 3: return launch_dma_bf16<XF32, 32, 32>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+    case 4: return launch_dma_bf16<XF32, 16, 64>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+    default: return launch_dma_bf16<XF32, 16, 32>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+    }
+}
+
 }  // namespace
 
 hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const uint16_t* w, int N,
@@ -407,12 +694,11 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
                                N, K, gelu, accumulate);
         return hipGetLastError();
     }
-    // 64x64 tiles when they give at least 256 workgroups, otherwise 32x32
-    // (M <= 32: norm_out's 6144 columns; proj_out's 64 columns); K of at
-    // most 256 (img_in) without the split of K over the waves
     const int64_t big = static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64);
-    if (K <= 256 && big >= 256) {
-        const int tiles = static_cast<int>(big);
+    // K of at most 256 (img_in) with enough tiles to fill the chip: no split
+    // of K over the waves
+    if (K <= 256 && big >= 256 && N <= kShortKMaxN) {
+        const int tiles = ((M + SK_M - 1) / SK_M) * ((N + SK_N - 1) / SK_N);
 #define QIMG_SHORTK(XF, GL)                                                                                    \
     hipLaunchKernelGGL((gemm_bf16_shortk_kernel<XF, GL>), dim3(tiles), dim3(BF_THR), 0, stream, x, w, bias, out, M, \
                        N, K, accumulate)
@@ -430,6 +716,11 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
 #undef QIMG_SHORTK
         return hipGetLastError();
     }
+    if (K % 128 == 0)
+        return xf32 ? launch_best_dma_bf16<true>(x, M, K, w, N, bias, out, gelu, accumulate, stream)
+                    : launch_best_dma_bf16<false>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+    // other K: direct fragment loads, 64x64 tiles when they give at least
+    // 256 workgroups, otherwise 32x32
     if (M > 32 && big >= 256)
         return xf32 ? launch_tiled_bf16<true, 2, 2>(x, M, K, w, N, bias, out, gelu, accumulate, stream)
                     : launch_tiled_bf16<false, 2, 2>(x, M, K, w, N, bias, out, gelu, accumulate, stream);

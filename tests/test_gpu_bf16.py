@@ -152,3 +152,17 @@ def test_linear_bf16_rejects_bad_arguments(qimg):
         qimg.linear_forward_bf16(x, torch.zeros(8, 32, dtype=torch.bfloat16, device=DEV))  # K mismatch
     L = qimg.lib()
     assert L.qimg_linear_bf16(qimg._ptr(x), 2, 4, 64, qimg._ptr(w), 8, None, qimg._ptr(x), 0, None) == 1  # fp16 x
+
+
+# tiles of 64, 32 and 16 rows and of 64 and 32 columns (whichever the byte
+# rule picks), last tiles of one row or column, N not a multiple of 4, one
+# stage of K and fewer stages than the ring holds; short K on 64 x 128 tiles
+DMA = [(1, 1, 128), (17, 61, 128), (15, 33, 256), (65, 4097, 384), (129, 6145, 512), (1025, 67, 3072),
+       (4097, 32, 1152), (300, 3074, 3584), (1000, 3000, 1024), (4096, 16, 3072), (16385, 64, 256),
+       (1025, 3075, 64), (4095, 1027, 32), (2049, 2051, 224)]
+
+
+@pytest.mark.parametrize("M,N,K", DMA)
+@pytest.mark.parametrize("x_fp32", [True, False])
+def test_linear_bf16_tile_edges_exact(qimg, oracle, M, N, K, x_fp32):
+    test_linear_bf16_integer_operands_exact(qimg, oracle, M, N, K, x_fp32)
