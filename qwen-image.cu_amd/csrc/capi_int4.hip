@@ -186,7 +186,8 @@ int qimg_linear_int4(const float* x, int M, const qimg_int4_weight* w, const uin
         e = qimg::launch_quant_act_int4(x, w->smooth, xs, base + L.a, reinterpret_cast<float*>(base + L.act_scales), M,
                                         K, gs, s);
     else
-        e = qimg::launch_int4_prep(x, w->smooth, xs, reinterpret_cast<uint16_t*>(base + L.xr), M, K, hbs, s);
+        e = qimg::launch_int4_prep(x, w->smooth, xs, hbs > 1 ? reinterpret_cast<uint16_t*>(base + L.xr) : nullptr, M,
+                                   K, hbs, s);
     if (e != hipSuccess) return api_hip_status(e, fn);
     // 2. low-rank branch: lr = bf16(x_lr . svd_down), out = lr . svd_up^T
     const bool fused = w4a4 && r > 0 && r % 16 == 0;  // the W4A4 kernel multiplies by svd_up itself
@@ -195,8 +196,7 @@ int qimg_linear_int4(const float* x, int M, const qimg_int4_weight* w, const uin
         float* lr32 = reinterpret_cast<float*>(base + L.lr32);
         uint16_t* lr16 = reinterpret_cast<uint16_t*>(base + L.lr16);
         if ((e = qimg::launch_transpose_u16(w->svd_down, svd_t, K, r, s)) != hipSuccess ||
-            (e = qimg::launch_linear_bf16(xs, QIMG_BF16, M, K, svd_t, r, nullptr, lr32, 0, s)) != hipSuccess ||
-            (e = qimg::launch_f32_to_bf16(lr32, lr16, static_cast<int64_t>(M) * r, s)) != hipSuccess ||
+            (e = qimg::launch_linear_bf16_out16(xs, M, K, svd_t, r, lr16, lr32, s)) != hipSuccess ||
             (!fused && (e = qimg::launch_linear_bf16(lr16, QIMG_BF16, M, r, w->svd_up, N, nullptr, out, 0, s)) !=
                            hipSuccess))
             return api_hip_status(e, fn);
@@ -211,8 +211,10 @@ int qimg_linear_int4(const float* x, int M, const qimg_int4_weight* w, const uin
         uint16_t* deq = reinterpret_cast<uint16_t*>(base + L.a);
         e = nk16 ? qimg::launch_dequant_int4_bf16(w->qweight, w->scales4, deq, N, K, gs, 0, 1, 1, s)
                  : qimg::launch_dequant_int4_bf16(w->qweight, w->scales4, deq, N, K, gs, w->nf4_grid != 0, 0, 0, s);
+        // without a rotation the residual's input is the low-rank one's
+        const uint16_t* xr = hbs > 1 ? reinterpret_cast<const uint16_t*>(base + L.xr) : xs;
         if (e == hipSuccess)
-            e = qimg::launch_linear_bf16(reinterpret_cast<const uint16_t*>(base + L.xr), QIMG_BF16, M, K, deq, N,
+            e = qimg::launch_linear_bf16(xr, QIMG_BF16, M, K, deq, N,
                                          bias_bf16, out, gelu != 0, s, r > 0);
     }
     return api_hip_status(e, fn);

@@ -401,7 +401,8 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __
 // wave is done with stage s - 1, whose slot is refilled right after.
 // LDS chunk c of row r sits at c ^ (r & 15): the 16 rows of a fragment read
 // fall on 16 different bank groups.
-// Rows past M and N re-read the last row and are not stored.
+// Rows past M and N re-read the last row and are not stored. With out16 the
+// result is rounded to bf16 there (out is not touched).
 // Measured against gemm_bf16_kernel (us, fp32 x): txt_in 256x3072x3584 48 ->
 // 24, proj_out 4096x64x3072 25 -> 11 (50 MB of x: 4.6 TB/s), norm_out
 // 1x6144x3072 11 -> 7.9 (38 MB of w: 4.8 TB/s); the INT4 down factor
@@ -424,8 +425,9 @@ struct BfDma {
 template <bool XF32, int TM, int TN, bool GELU>
 __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __restrict__ X,
                                                                const uint16_t* __restrict__ Wt,
-                                                               const uint16_t* __restrict__ bias, float* out, int M,
-                                                               int N, int K, int accumulate) {
+                                                               const uint16_t* __restrict__ bias, float* out,
+                                                               uint16_t* out16, int M, int N, int K,
+                                                               int accumulate) {
     using G = BfDma<XF32, TM, TN>;
     constexpr int NS = G::NS, PER = G::PER, XI = G::XI;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * G::STAGE];
@@ -575,7 +577,12 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __res
             if (GELU) t = gelu_tanh(t);
             v[c] = t;
         }
-        if (vec_ok) {
+        if (out16 != nullptr) {
+            uint16_t* o16 = out16 + static_cast<int64_t>(m) * N + col;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (col + c < N) o16[c] = f32_to_bf16(v[c]);
+        } else if (vec_ok) {
             *reinterpret_cast<v4f*>(o) = (v4f){v[0], v[1], v[2], v[3]};
         } else {
 #pragma unroll
@@ -630,14 +637,14 @@ hipError_t launch_tiled_bf16(const void* x, int M, int K, const uint16_t* w, int
 
 template <bool XF32, int TM, int TN>
 hipError_t launch_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N, const uint16_t* bias, float* out,
-                           int gelu, int accumulate, hipStream_t stream) {
+                           uint16_t* out16, int gelu, int accumulate, hipStream_t stream) {
     const int tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     if (gelu)
         hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, true>), dim3(tiles), dim3(BF_THR), 0, stream, x, w,
-                           bias, out, M, N, K, accumulate);
+                           bias, out, out16, M, N, K, accumulate);
     else
         hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, false>), dim3(tiles), dim3(BF_THR), 0, stream, x, w,
-                           bias, out, M, N, K, accumulate);
+                           bias, out, out16, M, N, K, accumulate);
     return hipGetLastError();
 }
 
@@ -646,7 +653,7 @@ hipError_t launch_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N
 // workgroups times the bytes of a tile's rows.
 template <bool XF32>
 hipError_t launch_best_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N, const uint16_t* bias,
-                                float* out, int gelu, int accumulate, hipStream_t stream) {
+                                float* out, uint16_t* out16, int gelu, int accumulate, hipStream_t stream) {
     constexpr int tm[] = {64, 64, 32, 32, 16, 16}, tn[] = {64, 32, 64, 32, 64, 32};
     int best = 0;
     int64_t best_cost = INT64_MAX;
@@ -659,12 +666,12 @@ hipError_t launch_best_dma_bf16(const void* x, int M, int K, const uint16_t* w, 
         }
     }
     switch (best) {
-    case 0: return launch_dma_bf16<XF32, 64, 64>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
-    case 1: return launch_dma_bf16<XF32, 64, 32>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
-    case 2: return launch_dma_bf16<XF32, 32, 64>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
-    case 3: return launch_dma_bf16<XF32, 32, 32>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
-    case 4: return launch_dma_bf16<XF32, 16, 64>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
-    default: return launch_dma_bf16<XF32, 16, 32>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+    case 0: return launch_dma_bf16<XF32, 64, 64>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
+    case 1: return launch_dma_bf16<XF32, 64, 32>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
+    case 2: return launch_dma_bf16<XF32, 32, 64>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
+    case 3: return launch_dma_bf16<XF32, 32, 32>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
+    case 4: return launch_dma_bf16<XF32, 16, 64>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
+    default: return launch_dma_bf16<XF32, 16, 32>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
     }
 }
 
@@ -717,8 +724,8 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
         return hipGetLastError();
     }
     if (K % 128 == 0)
-        return xf32 ? launch_best_dma_bf16<true>(x, M, K, w, N, bias, out, gelu, accumulate, stream)
-                    : launch_best_dma_bf16<false>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+        return xf32 ? launch_best_dma_bf16<true>(x, M, K, w, N, bias, out, nullptr, gelu, accumulate, stream)
+                    : launch_best_dma_bf16<false>(x, M, K, w, N, bias, out, nullptr, gelu, accumulate, stream);
     // other K: direct fragment loads, 64x64 tiles when they give at least
     // 256 workgroups, otherwise 32x32
     if (M > 32 && big >= 256)
@@ -726,6 +733,15 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
                     : launch_tiled_bf16<false, 2, 2>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
     return xf32 ? launch_tiled_bf16<true, 1, 1>(x, M, K, w, N, bias, out, gelu, accumulate, stream)
                 : launch_tiled_bf16<false, 1, 1>(x, M, K, w, N, bias, out, gelu, accumulate, stream);
+}
+
+hipError_t launch_linear_bf16_out16(const uint16_t* x, int M, int K, const uint16_t* w, int N, uint16_t* out,
+                                    float* tmp, hipStream_t stream) {
+    if (M == 0 || N == 0) return hipSuccess;
+    if (K > 0 && K % 128 == 0 && N <= 256)  // (wider ones may suit the 256x256 tiles)
+        return launch_best_dma_bf16<false>(x, M, K, w, N, nullptr, nullptr, out, 0, 0, stream);
+    const hipError_t e = launch_linear_bf16(x, QIMG_BF16, M, K, w, N, nullptr, tmp, 0, stream);
+    return e == hipSuccess ? launch_f32_to_bf16(tmp, out, static_cast<int64_t>(M) * N, stream) : e;
 }
 
 }  // namespace qimg

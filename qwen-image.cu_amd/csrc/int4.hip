@@ -28,40 +28,48 @@ __constant__ float kNf4Grid[16] = {-1.0f,   -0.6962f, -0.5251f, -0.3949f, -0.284
 
 __device__ __forceinline__ int nib_signed(int n) { return n >= 8 ? n - 16 : n; }
 
-__device__ __forceinline__ float dequant_nibble(int n, float s, int nf4, int signed_int4) {
-    if (nf4) return kNf4Grid[n] * s;
-    if (signed_int4) return static_cast<float>(nib_signed(n)) * s;
-    return static_cast<float>(n - 8) * s;
+// Value of code n before its scale.
+__device__ __forceinline__ float int4_code(int n, int nf4, int signed_int4) {
+    if (nf4) return kNf4Grid[n];
+    return static_cast<float>(signed_int4 ? nib_signed(n) : n - 8);
 }
 
 // dequantize_int4_to_bf16_kernel (cuda_kernels.cu:2876-2917): one thread per
-// 4 packed bytes (8 columns, one 16-byte bf16 store). K % 8 == 0.
-__global__ __launch_bounds__(256) void dequant_int4_bf16_kernel(const uint8_t* __restrict__ qw,
-                                                                const float* __restrict__ scales,
-                                                                uint16_t* __restrict__ out, int N, int K, int gs,
-                                                                int nf4, int scales_gn, int signed_int4) {
-    const int64_t words = static_cast<int64_t>(N) * (K / 8);
+// 4 packed bytes (8 columns, one 16-byte bf16 store), K % 8 == 0, nb blocks of
+// threads along a row and a stride of gridDim.x / nb rows. Bound by writing
+// the output: a byte's two code values come from an LDS table (grid lookups
+// from constant memory and 64-bit divisions per thread had made it 13.5 us at
+// 3072 x 3072, 1.7 TB/s; now 9.4 us).
+constexpr int ROW_THR = 128;
+__global__ __launch_bounds__(ROW_THR) void dequant_int4_bf16_kernel(const uint8_t* __restrict__ qw,
+                                                                    const float* __restrict__ scales,
+                                                                    uint16_t* __restrict__ out, int N, int K, int gs,
+                                                                    int nf4, int scales_gn, int signed_int4, int nb) {
+    __shared__ float2 table[256];
+    for (int i = threadIdx.x; i < 256; i += ROW_THR)
+        table[i] = make_float2(int4_code(i & 15, nf4, signed_int4), int4_code(i >> 4, nf4, signed_int4));
+    __syncthreads();
     const int G = K / gs;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < words;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const int row = static_cast<int>(i / (K / 8));
-        const int c0 = static_cast<int>(i % (K / 8)) * 8;
-        const uint32_t w = reinterpret_cast<const uint32_t*>(qw)[i];
+    const int word = (blockIdx.x % nb) * ROW_THR + threadIdx.x;
+    const int c0 = word * 8;
+    if (c0 >= K) return;
+    const int g0 = c0 / gs;
+    const bool one = (c0 + 7) / gs == g0;  // one group for the 8 columns
+    for (int row = blockIdx.x / nb; row < N; row += gridDim.x / nb) {
+        const uint32_t w = reinterpret_cast<const uint32_t*>(qw + static_cast<int64_t>(row) * (K / 2))[word];
+        auto scale = [&](int g) {
+            return scales_gn ? scales[static_cast<int64_t>(g) * N + row] : scales[static_cast<int64_t>(row) * G + g];
+        };
+        const float s = scale(g0);
         u32x4 o;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            float v[2];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int c = c0 + 2 * p + e;
-                const int g = c / gs;
-                const float s = scales_gn ? scales[static_cast<int64_t>(g) * N + row]
-                                          : scales[static_cast<int64_t>(row) * G + g];
-                v[e] = dequant_nibble((w >> (8 * p + 4 * e)) & 0xF, s, nf4, signed_int4);
-            }
-            o[p] = static_cast<uint32_t>(f32_to_bf16(v[0])) | (static_cast<uint32_t>(f32_to_bf16(v[1])) << 16);
+            const float2 t = table[(w >> (8 * p)) & 0xff];
+            const float s0 = one ? s : scale((c0 + 2 * p) / gs);
+            const float s1 = one ? s : scale((c0 + 2 * p + 1) / gs);
+            o[p] = pack_bf16x2(t.x * s0, t.y * s1);
         }
-        reinterpret_cast<u32x4*>(out)[i] = o;
+        reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * K)[word] = o;
     }
 }
 
@@ -113,48 +121,67 @@ __global__ __launch_bounds__(256) void quant_int4_weight_kernel(const float* __r
 
 // Activation INT4 quant (quantize_activation_int4_kernel, cuda_kernels.cu:
 // 3575-3636; with a smooth divide and a bf16 copy, fused_smooth_bf16_quant_
-// kernel, :3650-3705). A thread owns one column pair; a group of gs columns
-// is gs/2 consecutive lanes of one wave (gs = 32, 64 or 128), reduced with
-// lane exchanges. scales [G, M].
+// kernel, :3650-3705). A thread owns 8 columns of a row (32 bytes in, 16 and 4
+// out), nb blocks of threads along a row and a stride of gridDim.x / nb rows;
+// a group of gs columns is gs/8 consecutive lanes of one wave (gs = 32, 64 or
+// 128), reduced with lane exchanges. scales [G, M]. Bound by HBM, the IEEE
+// divisions next; with 2 columns a thread, a 64-bit division per thread and
+// 1-byte stores 4352 x 3072 took 33.9 us (2.5 TB/s), now 20.2 us (4.3 TB/s).
 template <int GS>
-__global__ __launch_bounds__(256) void quant_act_int4_kernel(const float* __restrict__ x,
-                                                             const float* __restrict__ smooth,
-                                                             uint16_t* __restrict__ bf16_out,
-                                                             uint8_t* __restrict__ packed,
-                                                             float* __restrict__ scales, int M, int K) {
-    constexpr int L = GS / 2;  // lanes per group
-    const int64_t pairs = static_cast<int64_t>(M) * (K / 2);
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    // every lane takes part in the exchanges; lanes past the end hold zeros
-    const bool live = t < pairs;
-    const int64_t tt = live ? t : 0;
-    const int64_t m = tt / (K / 2);
-    const int c = static_cast<int>(tt % (K / 2)) * 2;
-    float v0 = 0.0f, v1 = 0.0f;
-    if (live) {
-        const float2 xv = *reinterpret_cast<const float2*>(x + m * K + c);
-        v0 = xv.x;
-        v1 = xv.y;
-        if (smooth != nullptr) {
-            v0 = v0 / smooth[c];
-            v1 = v1 / smooth[c + 1];
-        }
-        if (bf16_out != nullptr)
-            *reinterpret_cast<uint32_t*>(bf16_out + m * K + c) =
-                static_cast<uint32_t>(f32_to_bf16(v0)) | (static_cast<uint32_t>(f32_to_bf16(v1)) << 16);
-    }
-    float amax = fmaxf(fabsf(v0), fabsf(v1));
+__global__ __launch_bounds__(ROW_THR) void quant_act_int4_kernel(const float* __restrict__ x,
+                                                                 const float* __restrict__ smooth,
+                                                                 uint16_t* __restrict__ bf16_out,
+                                                                 uint8_t* __restrict__ packed,
+                                                                 float* __restrict__ scales, int M, int K, int nb) {
+    const int c = ((blockIdx.x % nb) * ROW_THR + static_cast<int>(threadIdx.x)) * 8;
+    // every lane takes part in the exchanges; lanes past the row hold zeros
+    const bool live = c < K;
+    float sm[8];
+    if (smooth != nullptr && live) {
 #pragma unroll
-    for (int off = 1; off < L; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
-    if (!live) return;
-    const int g = c / GS;
-    if ((c % GS) == 0) scales[static_cast<int64_t>(g) * M + m] = amax / 7.0f;
-    const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
-    int q0 = static_cast<int>(roundf(v0 * inv));
-    int q1 = static_cast<int>(roundf(v1 * inv));
-    q0 = q0 < -7 ? -7 : (q0 > 7 ? 7 : q0);
-    q1 = q1 < -7 ? -7 : (q1 > 7 ? 7 : q1);
-    packed[m * (K / 2) + c / 2] = static_cast<uint8_t>((q0 & 0xF) | ((q1 & 0xF) << 4));
+        for (int h = 0; h < 2; ++h) {
+            const v4f t = reinterpret_cast<const v4f*>(smooth + c)[h];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sm[4 * h + e] = t[e];
+        }
+    }
+    for (int m = blockIdx.x / nb; m < M; m += gridDim.x / nb) {
+        float v[8] = {};
+        if (live) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const v4f t = reinterpret_cast<const v4f*>(x + static_cast<int64_t>(m) * K + c)[h];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[4 * h + e] = t[e];
+            }
+            if (smooth != nullptr) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = v[e] / sm[e];
+            }
+            if (bf16_out != nullptr) {
+                u32x4 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(v[2 * e], v[2 * e + 1]);
+                *reinterpret_cast<u32x4*>(bf16_out + static_cast<int64_t>(m) * K + c) = o;
+            }
+        }
+        float amax = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
+#pragma unroll
+        for (int off = 1; off < GS / 8; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
+        if (!live) continue;
+        if ((c % GS) == 0) scales[static_cast<int64_t>(c / GS) * M + m] = amax / 7.0f;
+        const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
+        uint32_t w = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            int q = static_cast<int>(roundf(v[e] * inv));
+            q = q < -7 ? -7 : (q > 7 ? 7 : q);
+            w |= static_cast<uint32_t>(q & 0xF) << (4 * e);
+        }
+        *reinterpret_cast<uint32_t*>(packed + static_cast<int64_t>(m) * (K / 2) + c / 2) = w;
+    }
 }
 
 // ---- W4A4 GEMM ---------------------------------------------------------
@@ -679,14 +706,20 @@ int grid_for(int64_t n, int per_block = 256) {
     return static_cast<int>(b < 65536 ? (b > 0 ? b : 1) : 65536);
 }
 
+// Workgroups of ROW_THR threads of 8 columns along a row.
+int row_blocks(int K) { return (K / 8 + ROW_THR - 1) / ROW_THR; }
+
 }  // namespace
 
 hipError_t launch_dequant_int4_bf16(const uint8_t* qw, const float* scales, uint16_t* out, int N, int K, int gs,
                                     int nf4, int scales_gn, int signed_int4, hipStream_t stream) {
     if (N == 0 || K == 0) return hipSuccess;
     if (K % 8 != 0 || gs <= 0 || K % gs != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(dequant_int4_bf16_kernel, dim3(grid_for(static_cast<int64_t>(N) * (K / 8))), dim3(256), 0,
-                       stream, qw, scales, out, N, K, gs, nf4, scales_gn, signed_int4);
+    // about 4096 workgroups: each loads its table for a few rows
+    const int nb = row_blocks(K);
+    const int rows = nb < 4096 ? 4096 / nb : 1;
+    hipLaunchKernelGGL(dequant_int4_bf16_kernel, dim3(static_cast<unsigned>(nb) * (N < rows ? N : rows)), dim3(ROW_THR),
+                       0, stream, qw, scales, out, N, K, gs, nf4, scales_gn, signed_int4, nb);
     return hipGetLastError();
 }
 
@@ -708,22 +741,23 @@ hipError_t launch_quant_act_int4(const float* x, const float* smooth, uint16_t* 
                                  float* scales, int M, int K, int gs, hipStream_t stream) {
     if (M == 0 || K == 0) return hipSuccess;
     if (K % gs != 0) return hipErrorInvalidValue;
-    const int64_t pairs = static_cast<int64_t>(M) * (K / 2);
-    const int64_t blocks64 = (pairs + 255) / 256;
-    if (blocks64 > 0x7fffffff) return hipErrorInvalidValue;
-    const int blocks = static_cast<int>(blocks64);
+    // one workgroup per row part, up to 2^23 of them (a launch holds fewer
+    // than 2^32 threads); past that they stride over the rows
+    const int nb = row_blocks(K);
+    const int rows = nb < (1 << 23) ? (1 << 23) / nb : 1;
+    const dim3 grid(static_cast<unsigned>(nb) * (M < rows ? M : rows));
     switch (gs) {
         case 32:
-            hipLaunchKernelGGL(quant_act_int4_kernel<32>, dim3(blocks), dim3(256), 0, stream, x, smooth, bf16_out,
-                               packed, scales, M, K);
+            hipLaunchKernelGGL(quant_act_int4_kernel<32>, grid, dim3(ROW_THR), 0, stream, x, smooth, bf16_out, packed,
+                               scales, M, K, nb);
             break;
         case 64:
-            hipLaunchKernelGGL(quant_act_int4_kernel<64>, dim3(blocks), dim3(256), 0, stream, x, smooth, bf16_out,
-                               packed, scales, M, K);
+            hipLaunchKernelGGL(quant_act_int4_kernel<64>, grid, dim3(ROW_THR), 0, stream, x, smooth, bf16_out, packed,
+                               scales, M, K, nb);
             break;
         case 128:
-            hipLaunchKernelGGL(quant_act_int4_kernel<128>, dim3(blocks), dim3(256), 0, stream, x, smooth, bf16_out,
-                               packed, scales, M, K);
+            hipLaunchKernelGGL(quant_act_int4_kernel<128>, grid, dim3(ROW_THR), 0, stream, x, smooth, bf16_out,
+                               packed, scales, M, K, nb);
             break;
         default:
             return hipErrorInvalidValue;

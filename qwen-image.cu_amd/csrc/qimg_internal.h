@@ -128,6 +128,10 @@ hipError_t launch_dequant_bias(const int32_t* acc, const float* as, const float*
 // accumulate != 0: out = out + x . w^T, then the bias and GELU
 hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const uint16_t* w, int N,
                               const uint16_t* bias, float* out, int gelu, hipStream_t stream, int accumulate = 0);
+// The same with bf16 x, no bias, and the fp32 sums rounded to bf16; tmp
+// [M, N] is used where K is not a multiple of 128 or N is above 256.
+hipError_t launch_linear_bf16_out16(const uint16_t* x, int M, int K, const uint16_t* w, int N, uint16_t* out,
+                                    float* tmp, hipStream_t stream);
 
 // gemm_w8a8.hip: the same product for bf16 x with the 256x256 tiles of the
 // quantized linear (K % 64 == 0); launch_linear_bf16 takes it when the
@@ -162,7 +166,8 @@ hipError_t launch_transpose_u16(const uint16_t* in, uint16_t* out, int R, int C,
 hipError_t launch_f32_to_bf16(const float* in, uint16_t* out, int64_t n, hipStream_t stream);
 hipError_t launch_bf16_to_f32(const uint16_t* in, float* out, int64_t n, hipStream_t stream);
 // Rows of x fp32 [M, K]: v = x (/ smooth[k]); xs_bf16 = bf16(v) (if
-// non-null); xr_bf16 = bf16(FWHT_hbs(v)) (hbs > 1; hbs <= 1: bf16(v)).
+// non-null); xr_bf16 = bf16(FWHT_hbs(v)) (hbs > 1; hbs <= 1: bf16(v)), or
+// null for xs_bf16 alone (K % 8 == 0).
 hipError_t launch_int4_prep(const float* x, const float* smooth, uint16_t* xs_bf16, uint16_t* xr_bf16, int M, int K,
                             int hbs, hipStream_t stream);
 // out = FWHT_hbs(x / smooth[k]) fp32 (smooth may be null, hbs <= 1: no

@@ -359,3 +359,27 @@ def test_linear_int4_rejects_bad_arguments(qimg):
     import ctypes
     assert L.qimg_linear_int4(qimg._ptr(x), 4, ctypes.byref(st), None, qimg._ptr(x), 0, qimg._ptr(scratch), 16,
                               None) == 3  # scratch too small
+
+
+@pytest.mark.parametrize("M,K,gs,smooth", [(5, 32, 32, True), (3, 1056, 32, True), (2, 1152, 128, False),
+                                           (131, 1024, 64, True), (1, 2112, 64, True)])
+def test_quantize_activation_int4_row_parts_bit_exact(qimg, oracle, M, K, gs, smooth):
+    """Rows around the 1024 columns a workgroup of the quantizer takes."""
+    test_quantize_activation_int4_bit_exact(qimg, oracle, M, K, gs, smooth)
+
+
+@pytest.mark.parametrize("N,K,gs", [(3, 1032, 8), (2, 1024, 64), (1400, 1040, 16), (5, 96, 6), (4097, 8, 8)])
+@pytest.mark.parametrize("form", ["nf4", "linear", "signed_gn"])
+def test_dequant_int4_row_parts_bit_exact(qimg, oracle, N, K, gs, form):
+    """Rows around 1024 columns, groups that end inside 8 columns, and more
+    rows than one pass of the grid."""
+    test_dequant_int4_bit_exact(qimg, oracle, N, K, gs, form)
+
+
+@pytest.mark.parametrize("M,K,hbs,smooth", [(1, 1024, 1024, True), (5, 2048, 1024, True), (6, 3072, 1024, False),
+                                            (7, 4096, 1024, True), (3, 12288, 4096, True), (4, 96, 32, True),
+                                            (9, 1000, 1, True)])
+def test_linear_int4_input_forms(qimg, oracle, M, K, hbs, smooth):
+    """The residual's input on the wave-per-row and workgroup-per-row
+    transforms and without one (rows not a multiple of a workgroup's four)."""
+    test_linear_int4(qimg, oracle, M, 64, K, 0, 8, False, smooth, False, hbs, False)
