@@ -59,6 +59,25 @@ Int4Layout int4_layout(int M, int K, int N, int r, int group_size, bool w4a4) {
     return L;
 }
 
+// W4A16 with the low-rank product inside the residual's: the input and the
+// dequantized weight are `pad` columns wider, [rotated x | lr] . [W | up]^T.
+// The transposed down factor is in the weight's place until the weight is
+// dequantized; without a rotation the low-rank input is xr itself (xs < 0).
+struct Int4ExtLayout {
+    int64_t a, xr, xs, total;
+};
+
+Int4ExtLayout int4_ext_layout(int M, int K, int N, int r, int pad, bool rotated) {
+    Int4ExtLayout L{};
+    const int64_t ld = static_cast<int64_t>(K) + pad;
+    L.a = 0;
+    L.xr = align256(std::max(N * ld * 2, static_cast<int64_t>(r) * K * 2));
+    L.xs = L.xr + align256(M * ld * 2);
+    L.total = L.xs + (rotated ? align256(static_cast<int64_t>(M) * K * 2) : 0);
+    if (!rotated) L.xs = -1;
+    return L;
+}
+
 // int4_scratch_bytes, cuda_kernels.cuh:475-487 (group size 64 assumed there)
 int64_t reference_int4_scratch(int M, int K, int N, int r) {
     const int64_t a16 = static_cast<int64_t>(N) * K * 2;
@@ -181,13 +200,38 @@ int qimg_linear_int4(const float* x, int M, const qimg_int4_weight* w, const uin
     uint8_t* base = static_cast<uint8_t*>(scratch);
     uint16_t* xs = reinterpret_cast<uint16_t*>(base + L.xs);
     hipError_t e;
+    // W4A16 with a low-rank branch, whole 128-column stages of K and the room
+    // for it: the low-rank product as `pad` more columns of the residual's (in
+    // the same fp32 sums) instead of a GEMM that writes [M, N] and a residual
+    // that reads it back. 64 columns a step on the 256x256 tiles, 128 below.
+    // 4096 x 3072 x 3072, rank 32: 14 us for the up GEMM and the residual's
+    // accumulate against 2 us for the longer K.
+    if (!w4a4 && r > 0 && qimg::linear_bf16_out16_direct(K, r)) {
+        const int step = qimg::linear_bf16_large(M, K, N) ? 64 : 128;
+        const int pad = (r + step - 1) / step * step;
+        const Int4ExtLayout X = int4_ext_layout(M, K, N, r, pad, hbs > 1);
+        if (scratch_bytes >= X.total) {
+            uint16_t* deq = reinterpret_cast<uint16_t*>(base + X.a);
+            uint16_t* xr = reinterpret_cast<uint16_t*>(base + X.xr);
+            uint16_t* in = hbs > 1 ? reinterpret_cast<uint16_t*>(base + X.xs) : xr;  // low-rank input
+            const int ld = K + pad, ldi = hbs > 1 ? K : ld;
+            e = qimg::launch_int4_prep(x, w->smooth, in, hbs > 1 ? xr : nullptr, M, K, hbs, pad, s);
+            if (e == hipSuccess) e = qimg::launch_transpose_u16(w->svd_down, deq, K, r, s);
+            if (e == hipSuccess) e = qimg::launch_linear_bf16_out16_ld(in, ldi, M, K, deq, r, xr + K, ld, s);
+            if (e == hipSuccess)
+                e = qimg::launch_dequant_int4_bf16_ext(w->qweight, w->scales4, deq, N, K, gs, !nk16 && w->nf4_grid,
+                                                       nk16, nk16, w->svd_up, r, pad, s);
+            if (e == hipSuccess) e = qimg::launch_linear_bf16(xr, QIMG_BF16, M, ld, deq, N, bias_bf16, out, gelu != 0, s);
+            return api_hip_status(e, fn);
+        }
+    }
     // 1. the inputs of both branches in one pass over x
     if (w4a4)
         e = qimg::launch_quant_act_int4(x, w->smooth, xs, base + L.a, reinterpret_cast<float*>(base + L.act_scales), M,
                                         K, gs, s);
     else
         e = qimg::launch_int4_prep(x, w->smooth, xs, hbs > 1 ? reinterpret_cast<uint16_t*>(base + L.xr) : nullptr, M,
-                                   K, hbs, s);
+                                   K, hbs, 0, s);
     if (e != hipSuccess) return api_hip_status(e, fn);
     // 2. low-rank branch: lr = bf16(x_lr . svd_down), out = lr . svd_up^T
     const bool fused = w4a4 && r > 0 && r % 16 == 0;  // the W4A4 kernel multiplies by svd_up itself

@@ -402,7 +402,8 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __
 // LDS chunk c of row r sits at c ^ (r & 15): the 16 rows of a fragment read
 // fall on 16 different bank groups.
 // Rows past M and N re-read the last row and are not stored. With out16 the
-// result is rounded to bf16 there (out is not touched).
+// result is rounded to bf16 there, rows of ldo (out is not touched). x has rows
+// of ldx.
 // Measured against gemm_bf16_kernel (us, fp32 x): txt_in 256x3072x3584 48 ->
 // 24, proj_out 4096x64x3072 25 -> 11 (50 MB of x: 4.6 TB/s), norm_out
 // 1x6144x3072 11 -> 7.9 (38 MB of w: 4.8 TB/s); the INT4 down factor
@@ -426,8 +427,8 @@ template <bool XF32, int TM, int TN, bool GELU>
 __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __restrict__ X,
                                                                const uint16_t* __restrict__ Wt,
                                                                const uint16_t* __restrict__ bias, float* out,
-                                                               uint16_t* out16, int M, int N, int K,
-                                                               int accumulate) {
+                                                               uint16_t* out16, int64_t ldx, int64_t ldo, int M,
+                                                               int N, int K, int accumulate) {
     using G = BfDma<XF32, TM, TN>;
     constexpr int NS = G::NS, PER = G::PER, XI = G::XI;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * G::STAGE];
@@ -461,7 +462,7 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __res
         const int c = ((off % rb) >> 4) ^ (row & 15);
         if (is_x) {
             const int gm = m0 + row < M ? m0 + row : M - 1;
-            src[j] = static_cast<const uint8_t*>(X) + static_cast<int64_t>(gm) * K * G::XE + c * 16;
+            src[j] = static_cast<const uint8_t*>(X) + gm * ldx * G::XE + c * 16;
         } else {
             const int gn = n0 + row < N ? n0 + row : N - 1;
             src[j] = reinterpret_cast<const uint8_t*>(Wt) + static_cast<int64_t>(gn) * K * 2 + c * 16;
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __res
             v[c] = t;
         }
         if (out16 != nullptr) {
-            uint16_t* o16 = out16 + static_cast<int64_t>(m) * N + col;
+            uint16_t* o16 = out16 + m * ldo + col;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
                 if (col + c < N) o16[c] = f32_to_bf16(v[c]);
@@ -637,14 +638,14 @@ hipError_t launch_tiled_bf16(const void* x, int M, int K, const uint16_t* w, int
 
 template <bool XF32, int TM, int TN>
 hipError_t launch_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N, const uint16_t* bias, float* out,
-                           uint16_t* out16, int gelu, int accumulate, hipStream_t stream) {
+                           uint16_t* out16, int64_t ldx, int64_t ldo, int gelu, int accumulate, hipStream_t stream) {
     const int tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     if (gelu)
         hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, true>), dim3(tiles), dim3(BF_THR), 0, stream, x, w,
-                           bias, out, out16, M, N, K, accumulate);
+                           bias, out, out16, ldx, ldo, M, N, K, accumulate);
     else
         hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, false>), dim3(tiles), dim3(BF_THR), 0, stream, x, w,
-                           bias, out, out16, M, N, K, accumulate);
+                           bias, out, out16, ldx, ldo, M, N, K, accumulate);
     return hipGetLastError();
 }
 
@@ -653,7 +654,8 @@ hipError_t launch_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N
 // workgroups times the bytes of a tile's rows.
 template <bool XF32>
 hipError_t launch_best_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N, const uint16_t* bias,
-                                float* out, uint16_t* out16, int gelu, int accumulate, hipStream_t stream) {
+                                float* out, uint16_t* out16, int64_t ldx, int64_t ldo, int gelu, int accumulate,
+                                hipStream_t stream) {
     constexpr int tm[] = {64, 64, 32, 32, 16, 16}, tn[] = {64, 32, 64, 32, 64, 32};
     int best = 0;
     int64_t best_cost = INT64_MAX;
@@ -666,16 +668,20 @@ hipError_t launch_best_dma_bf16(const void* x, int M, int K, const uint16_t* w, 
         }
     }
     switch (best) {
-    case 0: return launch_dma_bf16<XF32, 64, 64>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
-    case 1: return launch_dma_bf16<XF32, 64, 32>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
-    case 2: return launch_dma_bf16<XF32, 32, 64>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
-    case 3: return launch_dma_bf16<XF32, 32, 32>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
-    case 4: return launch_dma_bf16<XF32, 16, 64>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
-    default: return launch_dma_bf16<XF32, 16, 32>(x, M, K, w, N, bias, out, out16, gelu, accumulate, stream);
+    case 0: return launch_dma_bf16<XF32, 64, 64>(x, M, K, w, N, bias, out, out16, ldx, ldo, gelu, accumulate, stream);
+    case 1: return launch_dma_bf16<XF32, 64, 32>(x, M, K, w, N, bias, out, out16, ldx, ldo, gelu, accumulate, stream);
+    case 2: return launch_dma_bf16<XF32, 32, 64>(x, M, K, w, N, bias, out, out16, ldx, ldo, gelu, accumulate, stream);
+    case 3: return launch_dma_bf16<XF32, 32, 32>(x, M, K, w, N, bias, out, out16, ldx, ldo, gelu, accumulate, stream);
+    case 4: return launch_dma_bf16<XF32, 16, 64>(x, M, K, w, N, bias, out, out16, ldx, ldo, gelu, accumulate, stream);
+    default: return launch_dma_bf16<XF32, 16, 32>(x, M, K, w, N, bias, out, out16, ldx, ldo, gelu, accumulate, stream);
     }
 }
 
 }  // namespace
+
+bool linear_bf16_large(int M, int K, int N) {
+    return K % 64 == 0 && static_cast<int64_t>((M + 255) / 256) * ((N + 255) / 256) >= 128;
+}
 
 hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const uint16_t* w, int N,
                               const uint16_t* bias, float* out, int gelu, hipStream_t stream, int accumulate) {
@@ -685,8 +691,7 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
     const int64_t wbytes = static_cast<int64_t>(N) * K * 2;
     // Large problems with bf16 x (the INT4 linear's residual GEMM at 4096
     // tokens): the quantized linear's 256x256 tiles with bf16 MFMA.
-    const int64_t tiles256 = static_cast<int64_t>((M + 255) / 256) * ((N + 255) / 256);
-    if (!xf32 && (K % 64) == 0 && tiles256 >= 128)
+    if (!xf32 && linear_bf16_large(M, K, N))
         return launch_gemm_bf16_large(static_cast<const uint16_t*>(x), M, K, w, N, bias, out, gelu, accumulate,
                                       stream);
     const bool tiled = (K % BF_KB) == 0 && xbytes < (int64_t{1} << 31) && wbytes < (int64_t{1} << 31);
@@ -724,8 +729,8 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
         return hipGetLastError();
     }
     if (K % 128 == 0)
-        return xf32 ? launch_best_dma_bf16<true>(x, M, K, w, N, bias, out, nullptr, gelu, accumulate, stream)
-                    : launch_best_dma_bf16<false>(x, M, K, w, N, bias, out, nullptr, gelu, accumulate, stream);
+        return xf32 ? launch_best_dma_bf16<true>(x, M, K, w, N, bias, out, nullptr, K, N, gelu, accumulate, stream)
+                    : launch_best_dma_bf16<false>(x, M, K, w, N, bias, out, nullptr, K, N, gelu, accumulate, stream);
     // other K: direct fragment loads, 64x64 tiles when they give at least
     // 256 workgroups, otherwise 32x32
     if (M > 32 && big >= 256)
@@ -738,10 +743,19 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
 hipError_t launch_linear_bf16_out16(const uint16_t* x, int M, int K, const uint16_t* w, int N, uint16_t* out,
                                     float* tmp, hipStream_t stream) {
     if (M == 0 || N == 0) return hipSuccess;
-    if (K > 0 && K % 128 == 0 && N <= 256)  // (wider ones may suit the 256x256 tiles)
-        return launch_best_dma_bf16<false>(x, M, K, w, N, nullptr, nullptr, out, 0, 0, stream);
+    if (linear_bf16_out16_direct(K, N)) return launch_linear_bf16_out16_ld(x, K, M, K, w, N, out, N, stream);
     const hipError_t e = launch_linear_bf16(x, QIMG_BF16, M, K, w, N, nullptr, tmp, 0, stream);
     return e == hipSuccess ? launch_f32_to_bf16(tmp, out, static_cast<int64_t>(M) * N, stream) : e;
+}
+
+// (wider products may suit the 256x256 tiles)
+bool linear_bf16_out16_direct(int K, int N) { return K > 0 && K % 128 == 0 && N <= 256; }
+
+hipError_t launch_linear_bf16_out16_ld(const uint16_t* x, int64_t ldx, int M, int K, const uint16_t* w, int N,
+                                       uint16_t* out, int64_t ldo, hipStream_t stream) {
+    if (M == 0 || N == 0) return hipSuccess;
+    if (!linear_bf16_out16_direct(K, N)) return hipErrorInvalidValue;
+    return launch_best_dma_bf16<false>(x, M, K, w, N, nullptr, nullptr, out, ldx, ldo, 0, 0, stream);
 }
 
 }  // namespace qimg

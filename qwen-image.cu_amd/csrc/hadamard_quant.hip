@@ -755,10 +755,17 @@ __device__ __forceinline__ void smooth_chunk(const float* x, const float* __rest
 template <RowOut OUT>
 __global__ __launch_bounds__(256) void smooth_fwht_rows_kernel(const float* x, const float* __restrict__ smooth,
                                                                uint16_t* __restrict__ xs, void* xr, int K,
-                                                               int hbs_log2, float norm) {
+                                                               int hbs_log2, float norm, int pad) {
     extern __shared__ float lds[];
     float* red = lds + lds_pad(K) + 1;
     const int row = blockIdx.x;
+    if constexpr (OUT == RowOut::Bf16) {
+        // rows of K + pad: this row starts at row * K of the shifted pointer
+        uint16_t* o = static_cast<uint16_t*>(xr) + static_cast<int64_t>(row) * pad;
+        for (int i = threadIdx.x; i < pad / 8; i += blockDim.x)
+            reinterpret_cast<u32x4*>(o + (static_cast<int64_t>(row) + 1) * K)[i] = (u32x4){0u, 0u, 0u, 0u};
+        xr = o;
+    }
     const int64_t base = static_cast<int64_t>(row) * K;
     int lo = 0;
     if ((K & 15) == 0 && hbs_log2 > 4) {
@@ -791,7 +798,8 @@ __global__ __launch_bounds__(256) void smooth_fwht_rows_kernel(const float* x, c
 // 21.0 us here (4.8 TB/s).
 template <int NB>
 __global__ __launch_bounds__(256) void smooth_fwht_wave_rows_kernel(const float* x, const float* __restrict__ smooth,
-                                                                    uint16_t* xs, uint16_t* xr, int M, float norm) {
+                                                                    uint16_t* xs, uint16_t* xr, int M, float norm,
+                                                                    int pad) {
     constexpr int HBS = 1024;
     constexpr int PADDED = HBS + HBS / 16;
     constexpr int K = NB * HBS;
@@ -802,6 +810,7 @@ __global__ __launch_bounds__(256) void smooth_fwht_wave_rows_kernel(const float*
     if (row >= M) return;  // whole waves: no barrier below
     float* lds = lds_all + wave * PADDED;
     const int64_t base = static_cast<int64_t>(row) * K;
+    xr += base + static_cast<int64_t>(row) * pad;
     float v[NB][16];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -816,32 +825,40 @@ __global__ __launch_bounds__(256) void smooth_fwht_wave_rows_kernel(const float*
         float t[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) t[i] = lds[lds_pad(16 * lane + i)];
-        store_bf16x16(xr + base + b * HBS + 16 * lane, t);
+        store_bf16x16(xr + b * HBS + 16 * lane, t);
         wave_lds_order();
     }
+    for (int i = lane; i < pad / 8; i += 64) reinterpret_cast<u32x4*>(xr + K)[i] = (u32x4){0u, 0u, 0u, 0u};
 }
 
-// bf16(x / smooth) alone (no rotation): 8 columns a thread, K % 8 == 0.
+// bf16(x / smooth) alone (no rotation): 8 columns a thread, K % 8 == 0, rows
+// of per_row + pad8 chunks of 8, the last pad8 zeros.
 __global__ __launch_bounds__(256) void smooth_bf16_kernel(const float* __restrict__ x, const float* __restrict__ smooth,
-                                                          uint16_t* __restrict__ xs, int64_t chunks, int per_row) {
+                                                          uint16_t* __restrict__ xs, int64_t chunks, int per_row,
+                                                          int pad8) {
+    const int ld = per_row + pad8;
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < chunks;
          i += static_cast<int64_t>(gridDim.x) * 256) {
-        const v4f* p = reinterpret_cast<const v4f*>(x) + 2 * i;
-        v4f lo = p[0], hi = p[1];
-        if (smooth != nullptr) {
-            const v4f* sp = reinterpret_cast<const v4f*>(smooth) +
-                            2 * (chunks <= 0x7fffffff ? static_cast<int>(i) % per_row : static_cast<int>(i % per_row));
-            lo = lo / sp[0];
-            hi = hi / sp[1];
+        const int64_t row = chunks <= 0x7fffffff ? static_cast<int>(i) / ld : i / ld;
+        const int c = static_cast<int>(i - row * ld);
+        u32x4 o = {0u, 0u, 0u, 0u};
+        if (c < per_row) {
+            const v4f* p = reinterpret_cast<const v4f*>(x) + 2 * (row * per_row + c);
+            v4f lo = p[0], hi = p[1];
+            if (smooth != nullptr) {
+                lo = lo / reinterpret_cast<const v4f*>(smooth)[2 * c];
+                hi = hi / reinterpret_cast<const v4f*>(smooth)[2 * c + 1];
+            }
+            o = (u32x4){pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]),
+                        pack_bf16x2(hi[2], hi[3])};
         }
-        reinterpret_cast<u32x4*>(xs)[i] = (u32x4){pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]),
-                                                  pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+        reinterpret_cast<u32x4*>(xs)[i] = o;
     }
 }
 
 template <RowOut OUT>
 static hipError_t launch_smooth_fwht(const float* x, const float* smooth, uint16_t* xs, void* xr, int M, int K,
-                                     int hbs, hipStream_t stream) {
+                                     int hbs, int pad, hipStream_t stream) {
     if (M == 0 || K == 0) return hipSuccess;
     if (hbs < 1) hbs = 1;
     if ((hbs & (hbs - 1)) != 0 || K % hbs != 0) return hipErrorInvalidValue;
@@ -858,19 +875,20 @@ static hipError_t launch_smooth_fwht(const float* x, const float* smooth, uint16
     while ((1 << lg) < hbs) ++lg;
     const float norm = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(hbs)));
     hipLaunchKernelGGL(smooth_fwht_rows_kernel<OUT>, dim3(M), dim3(threads), lds, stream, x, smooth, xs, xr, K, lg,
-                       norm);
+                       norm, pad);
     return hipGetLastError();
 }
 
 hipError_t launch_int4_prep(const float* x, const float* smooth, uint16_t* xs_bf16, uint16_t* xr_bf16, int M, int K,
-                            int hbs, hipStream_t stream) {
+                            int hbs, int pad, hipStream_t stream) {
+    if (pad < 0 || pad % 8 != 0) return hipErrorInvalidValue;
     if (M == 0 || K == 0) return hipSuccess;
     if (xr_bf16 == nullptr) {
         if (K % 8 != 0) return hipErrorInvalidValue;
-        const int64_t chunks = static_cast<int64_t>(M) * (K / 8);
+        const int64_t chunks = static_cast<int64_t>(M) * ((K + pad) / 8);
         const int64_t blocks = (chunks + 255) / 256;
         hipLaunchKernelGGL(smooth_bf16_kernel, dim3(static_cast<unsigned>(blocks < 65536 ? blocks : 65536)), dim3(256),
-                           0, stream, x, smooth, xs_bf16, chunks, K / 8);
+                           0, stream, x, smooth, xs_bf16, chunks, K / 8, pad / 8);
         return hipGetLastError();
     }
     if (hbs == 1024 && K % 1024 == 0 && K / 1024 <= 4) {
@@ -879,29 +897,29 @@ hipError_t launch_int4_prep(const float* x, const float* smooth, uint16_t* xs_bf
         switch (K / 1024) {
             case 1:
                 hipLaunchKernelGGL(smooth_fwht_wave_rows_kernel<1>, grid, block, 0, stream, x, smooth, xs_bf16, xr_bf16,
-                                   M, norm);
+                                   M, norm, pad);
                 break;
             case 2:
                 hipLaunchKernelGGL(smooth_fwht_wave_rows_kernel<2>, grid, block, 0, stream, x, smooth, xs_bf16, xr_bf16,
-                                   M, norm);
+                                   M, norm, pad);
                 break;
             case 3:
                 hipLaunchKernelGGL(smooth_fwht_wave_rows_kernel<3>, grid, block, 0, stream, x, smooth, xs_bf16, xr_bf16,
-                                   M, norm);
+                                   M, norm, pad);
                 break;
             default:
                 hipLaunchKernelGGL(smooth_fwht_wave_rows_kernel<4>, grid, block, 0, stream, x, smooth, xs_bf16, xr_bf16,
-                                   M, norm);
+                                   M, norm, pad);
                 break;
         }
         return hipGetLastError();
     }
-    return launch_smooth_fwht<RowOut::Bf16>(x, smooth, xs_bf16, xr_bf16, M, K, hbs, stream);
+    return launch_smooth_fwht<RowOut::Bf16>(x, smooth, xs_bf16, xr_bf16, M, K, hbs, pad, stream);
 }
 
 hipError_t launch_smooth_fwht_f32(const float* x, const float* smooth, float* out, int M, int K, int hbs,
                                   hipStream_t stream) {
-    return launch_smooth_fwht<RowOut::Fp32>(x, smooth, nullptr, out, M, K, hbs, stream);
+    return launch_smooth_fwht<RowOut::Fp32>(x, smooth, nullptr, out, M, K, hbs, 0, stream);
 }
 
 // LayerNorm + modulate (ln_modulate_row) feeding the FWHT + row quant of

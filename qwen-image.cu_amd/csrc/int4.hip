@@ -37,14 +37,18 @@ __device__ __forceinline__ float int4_code(int n, int nf4, int signed_int4) {
 // dequantize_int4_to_bf16_kernel (cuda_kernels.cu:2876-2917): one thread per
 // 4 packed bytes (8 columns, one 16-byte bf16 store), K % 8 == 0, nb blocks of
 // threads along a row and a stride of gridDim.x / nb rows. Bound by writing
-// the output: a byte's two code values come from an LDS table (grid lookups
+// the output; the next row's words are loaded before this one's are used. With
+// pad > 0 a row of out is K + pad long, columns K .. K + r taken from up [N, r]
+// and the rest zero. A byte's two code values come from an LDS table (grid lookups
 // from constant memory and 64-bit divisions per thread had made it 13.5 us at
 // 3072 x 3072, 1.7 TB/s; now 9.4 us).
 constexpr int ROW_THR = 128;
 __global__ __launch_bounds__(ROW_THR) void dequant_int4_bf16_kernel(const uint8_t* __restrict__ qw,
                                                                     const float* __restrict__ scales,
                                                                     uint16_t* __restrict__ out, int N, int K, int gs,
-                                                                    int nf4, int scales_gn, int signed_int4, int nb) {
+                                                                    int nf4, int scales_gn, int signed_int4,
+                                                                    const uint16_t* __restrict__ up, int r, int pad,
+                                                                    int nb) {
     __shared__ float2 table[256];
     for (int i = threadIdx.x; i < 256; i += ROW_THR)
         table[i] = make_float2(int4_code(i & 15, nf4, signed_int4), int4_code(i >> 4, nf4, signed_int4));
@@ -52,24 +56,49 @@ __global__ __launch_bounds__(ROW_THR) void dequant_int4_bf16_kernel(const uint8_
     const int G = K / gs;
     const int word = (blockIdx.x % nb) * ROW_THR + threadIdx.x;
     const int c0 = word * 8;
-    if (c0 >= K) return;
+    const int64_t ldo = K + pad;
+    const int stride = gridDim.x / nb;
+    int row = blockIdx.x / nb;
+    if (c0 >= K) {
+        if (c0 >= ldo) return;
+        for (; row < N; row += stride) {
+            u32x4 o;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const int j = c0 - K + 2 * p;
+                const uint16_t* u = up + static_cast<int64_t>(row) * r + j;
+                o[p] = (j < r ? u[0] : 0u) | ((j + 1 < r ? static_cast<uint32_t>(u[1]) : 0u) << 16);
+            }
+            reinterpret_cast<u32x4*>(out + row * ldo)[word] = o;
+        }
+        return;
+    }
     const int g0 = c0 / gs;
     const bool one = (c0 + 7) / gs == g0;  // one group for the 8 columns
-    for (int row = blockIdx.x / nb; row < N; row += gridDim.x / nb) {
-        const uint32_t w = reinterpret_cast<const uint32_t*>(qw + static_cast<int64_t>(row) * (K / 2))[word];
-        auto scale = [&](int g) {
-            return scales_gn ? scales[static_cast<int64_t>(g) * N + row] : scales[static_cast<int64_t>(row) * G + g];
-        };
-        const float s = scale(g0);
+    auto code = [&](int n) {
+        return reinterpret_cast<const uint32_t*>(qw + static_cast<int64_t>(n) * (K / 2))[word];
+    };
+    auto scale = [&](int n, int g) {
+        return scales_gn ? scales[static_cast<int64_t>(g) * N + n] : scales[static_cast<int64_t>(n) * G + g];
+    };
+    uint32_t wn = row < N ? code(row) : 0u;
+    float sn = row < N ? scale(row, g0) : 0.0f;
+    for (; row < N; row += stride) {
+        const uint32_t w = wn;
+        const float s = sn;
+        if (row + stride < N) {
+            wn = code(row + stride);
+            sn = scale(row + stride, g0);
+        }
         u32x4 o;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             const float2 t = table[(w >> (8 * p)) & 0xff];
-            const float s0 = one ? s : scale((c0 + 2 * p) / gs);
-            const float s1 = one ? s : scale((c0 + 2 * p + 1) / gs);
+            const float s0 = one ? s : scale(row, (c0 + 2 * p) / gs);
+            const float s1 = one ? s : scale(row, (c0 + 2 * p + 1) / gs);
             o[p] = pack_bf16x2(t.x * s0, t.y * s1);
         }
-        reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * K)[word] = o;
+        reinterpret_cast<u32x4*>(out + row * ldo)[word] = o;
     }
 }
 
@@ -713,13 +742,19 @@ int row_blocks(int K) { return (K / 8 + ROW_THR - 1) / ROW_THR; }
 
 hipError_t launch_dequant_int4_bf16(const uint8_t* qw, const float* scales, uint16_t* out, int N, int K, int gs,
                                     int nf4, int scales_gn, int signed_int4, hipStream_t stream) {
+    return launch_dequant_int4_bf16_ext(qw, scales, out, N, K, gs, nf4, scales_gn, signed_int4, nullptr, 0, 0, stream);
+}
+
+hipError_t launch_dequant_int4_bf16_ext(const uint8_t* qw, const float* scales, uint16_t* out, int N, int K, int gs,
+                                        int nf4, int scales_gn, int signed_int4, const uint16_t* up, int r, int pad,
+                                        hipStream_t stream) {
     if (N == 0 || K == 0) return hipSuccess;
-    if (K % 8 != 0 || gs <= 0 || K % gs != 0) return hipErrorInvalidValue;
+    if (K % 8 != 0 || gs <= 0 || K % gs != 0 || pad < r || pad % 8 != 0) return hipErrorInvalidValue;
     // about 4096 workgroups: each loads its table for a few rows
-    const int nb = row_blocks(K);
+    const int nb = row_blocks(K + pad);
     const int rows = nb < 4096 ? 4096 / nb : 1;
     hipLaunchKernelGGL(dequant_int4_bf16_kernel, dim3(static_cast<unsigned>(nb) * (N < rows ? N : rows)), dim3(ROW_THR),
-                       0, stream, qw, scales, out, N, K, gs, nf4, scales_gn, signed_int4, nb);
+                       0, stream, qw, scales, out, N, K, gs, nf4, scales_gn, signed_int4, up, r, pad, nb);
     return hipGetLastError();
 }
 

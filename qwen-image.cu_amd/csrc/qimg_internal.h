@@ -132,6 +132,13 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
 // [M, N] is used where K is not a multiple of 128 or N is above 256.
 hipError_t launch_linear_bf16_out16(const uint16_t* x, int M, int K, const uint16_t* w, int N, uint16_t* out,
                                     float* tmp, hipStream_t stream);
+// The same where linear_bf16_out16_direct holds, with x in rows of ldx (a
+// multiple of 8) and out in rows of ldo.
+bool linear_bf16_out16_direct(int K, int N);
+hipError_t launch_linear_bf16_out16_ld(const uint16_t* x, int64_t ldx, int M, int K, const uint16_t* w, int N,
+                                       uint16_t* out, int64_t ldo, hipStream_t stream);
+// Whether launch_linear_bf16 takes the 256x256 tiles for bf16 x.
+bool linear_bf16_large(int M, int K, int N);
 
 // gemm_w8a8.hip: the same product for bf16 x with the 256x256 tiles of the
 // quantized linear (K % 64 == 0); launch_linear_bf16 takes it when the
@@ -142,6 +149,11 @@ hipError_t launch_gemm_bf16_large(const uint16_t* x, int M, int K, const uint16_
 // ---- INT4 paths (int4.hip, hadamard_quant.hip) ----
 hipError_t launch_dequant_int4_bf16(const uint8_t* qw, const float* scales, uint16_t* out, int N, int K, int gs,
                                     int nf4, int scales_gn, int signed_int4, hipStream_t stream);
+// The same into rows of K + pad (pad % 8 == 0): columns K .. K + r hold up
+// [N, r], the rest of the pad zeros.
+hipError_t launch_dequant_int4_bf16_ext(const uint8_t* qw, const float* scales, uint16_t* out, int N, int K, int gs,
+                                        int nf4, int scales_gn, int signed_int4, const uint16_t* up, int r, int pad,
+                                        hipStream_t stream);
 hipError_t launch_quant_int4_weight(const float* r, uint8_t* qw, float* scales, int N, int K, int gs, int nf4,
                                     hipStream_t stream);
 hipError_t launch_quant_act_int4(const float* x, const float* smooth, uint16_t* bf16_out, uint8_t* packed,
@@ -168,8 +180,10 @@ hipError_t launch_bf16_to_f32(const uint16_t* in, float* out, int64_t n, hipStre
 // Rows of x fp32 [M, K]: v = x (/ smooth[k]); xs_bf16 = bf16(v) (if
 // non-null); xr_bf16 = bf16(FWHT_hbs(v)) (hbs > 1; hbs <= 1: bf16(v)), or
 // null for xs_bf16 alone (K % 8 == 0).
+// With pad > 0 (pad % 8 == 0) the rows of xr_bf16 (of xs_bf16 where xr_bf16 is
+// null) are K + pad long and the pad is zeros.
 hipError_t launch_int4_prep(const float* x, const float* smooth, uint16_t* xs_bf16, uint16_t* xr_bf16, int M, int K,
-                            int hbs, hipStream_t stream);
+                            int hbs, int pad, hipStream_t stream);
 // out = FWHT_hbs(x / smooth[k]) fp32 (smooth may be null, hbs <= 1: no
 // transform); out may be x.
 hipError_t launch_smooth_fwht_f32(const float* x, const float* smooth, float* out, int M, int K, int hbs,

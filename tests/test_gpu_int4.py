@@ -383,3 +383,40 @@ def test_linear_int4_input_forms(qimg, oracle, M, K, hbs, smooth):
     """The residual's input on the wave-per-row and workgroup-per-row
     transforms and without one (rows not a multiple of a workgroup's four)."""
     test_linear_int4(qimg, oracle, M, 64, K, 0, 8, False, smooth, False, hbs, False)
+
+
+@pytest.mark.parametrize("M,N,K,r,hbs,smooth,nf4", [
+    (300, 1000, 1024, 20, 1024, True, True),      # r not a multiple of 8, ragged tiles
+    (130, 64, 3072, 130, 1024, False, True),      # r past one 128-column step
+    (260, 200, 128, 3, 1, True, False),           # one stage of K, no rotation
+    (2817, 3072, 256, 70, 256, True, True),       # the 256x256 tiles, r past one 64-column step
+    (150, 96, 4096, 1, 4096, False, False),
+])
+def test_linear_w4a16_low_rank_columns(qimg, oracle, M, N, K, r, hbs, smooth, nf4):
+    """The low-rank product as columns of the residual's product, against the
+    oracle, and against the separate low-rank GEMMs that a call with less
+    scratch takes: the same fp32 products in another order, so within 8
+    sqrt(K + r) 2^-24 of their absolute sum, itself below sqrt(K + r) times
+    the largest output (independent signs), plus a bf16 step of a low-rank
+    value whose fp32 sum lies on a rounding boundary (2^-8 of |lr| |up|)."""
+    test_linear_int4(qimg, oracle, M, N, K, r, 64, False, smooth, nf4, hbs, True)
+    rng = np.random.default_rng(M + r)
+    c = _int4_case(oracle, rng, M, N, K, r, 64, False, smooth, nf4, hbs)
+    bdev = lambda a: _bf16_bits_dev(a)
+    w = qimg.Int4Weight(N, K, 64, svd_up=bdev(c["up"]), svd_down=bdev(c["down"]), qweight=_u8(c["qw"]),
+                        scales4=_f32(c["s4"]), nf4_grid=nf4, had_block_size=hbs,
+                        smooth=_f32(c["sm"]) if smooth else None)
+    x = _f32(c["x"])
+    a = lambda n: (n + 255) // 256 * 256
+    least = a(max(N * K * 2, r * K * 2)) + 2 * a(M * K * 2) + a(M * r * 4) + a(M * r * 2)
+    got = qimg.linear_forward_int4(x, w)
+    sep = qimg.linear_forward_int4(x, w, scratch=torch.empty(least, dtype=torch.uint8, device=DEV))
+    torch.cuda.synchronize()
+    up = oracle.bf16_bits_to_f32(c["up"]).reshape(N, r)
+    down = oracle.bf16_bits_to_f32(c["down"]).reshape(K, r)
+    v = c["x"] / c["sm"] if smooth else c["x"]
+    lr_max = np.abs(v @ down).max()
+    bound = 8 * (K + r) * 2.0 ** -24 * float(sep.abs().max()) + 2.0 ** -8 * lr_max * np.abs(up).max()
+    assert float((got - sep).abs().max()) <= bound
+    with pytest.raises(qimg.QimgError):
+        qimg.linear_forward_int4(x, w, scratch=torch.empty(least - 256, dtype=torch.uint8, device=DEV))
