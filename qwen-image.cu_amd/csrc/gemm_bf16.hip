@@ -39,6 +39,7 @@ namespace {
 constexpr int BF_THR = 256;  // four waves, one K quarter each
 constexpr int BF_KB = 32;    // elements of K per block
 constexpr int SK_M = 64, SK_N = 128;  // tile of the short-K kernel
+constexpr int SK_XP = 72;  // bf16 per LDS row of 64 x values (16 rows fall on 16 bank groups)
 constexpr int kShortKMaxN = 1 << 22;  // its tile's output rows stay below 2^31 bytes (kOob out of range)
 constexpr int kRsrcWord3 = 0x00020000;  // raw unswizzled buffer (gfx9 family)
 constexpr uint32_t kOob = 0x80000000u;  // offset >= num_records: reads zero
@@ -254,14 +255,17 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_kernel(const void* __restric
 
 // Short K (img_in: K = 64): bound by writing the output. A workgroup owns 64
 // rows x 128 columns, each wave 64 x 32 (two 32x32 blocks), and runs the
-// whole of K, so no partial tiles are reduced; the operand loads and fragments
-// are those of gemm_bf16_kernel with x as the A operand, two K blocks loaded
-// at a time, the products summed in K-block order. Each block of 32 rows then
-// goes through LDS, so that a store instruction writes 512 contiguous bytes of
-// two rows. Tiles are numbered n first, so that workgroups in flight together
-// write whole output rows. 4096x3072x64: 29.9 us with 16-byte stores of 32
-// rows per instruction, 23.8 with 128-byte lines of two rows straight from
-// the accumulators, 21.6 as it is (50 MB: 2.3 TB/s).
+// whole of K, so no partial tiles are reduced; the fragments are those of
+// gemm_bf16_kernel with x as the A operand, the products summed in K-block
+// order. 64 k of the tile's x rows at a time come in whole lines, are rounded
+// to bf16 once and shared through LDS (every wave loading its own fp32
+// fragments, 32 lines an instruction, cost 7 us of 21); w goes straight to
+// fragments. The tile then goes through LDS, so that a store instruction
+// writes 512 contiguous bytes of two rows. Tiles are numbered n first, so that
+// workgroups in flight together write whole output rows. 4096x3072x64: 29.9
+// us with fragments and 16-byte stores of 32 rows per instruction, 21 with the
+// output through LDS, 11.8 with x through LDS too (51 MB: 4.3 TB/s; a fill of
+// the output alone takes 9.4 us); 6889 rows 16.8, K = 256 58 -> 22.5.
 template <bool XF32, bool GELU>
 __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __restrict__ X,
                                                                   const uint16_t* __restrict__ Wt,
@@ -269,7 +273,7 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __
                                                                   float* out, int M, int N, int K, int accumulate) {
     constexpr int XE = XF32 ? 4 : 2;
     constexpr int PITCH = SK_N + 4;
-    __shared__ __attribute__((aligned(16))) float stage[32 * PITCH];
+    __shared__ __attribute__((aligned(16))) float stage[SK_M * PITCH];
     const int tiles_m = (M + SK_M - 1) / SK_M;
     const int tiles_n = (N + SK_N - 1) / SK_N;
     const int logical = xcd_remap(blockIdx.x, tiles_m * tiles_n);
@@ -289,59 +293,61 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __
     // the tile's rows of out, those past M out of range
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
         out + static_cast<int64_t>(m0) * N, 0, (M - m0 < SK_M ? M - m0 : SK_M) * N * 4, kRsrcWord3);
-    uint32_t ox[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-        ox[i] = m0 + 32 * i + r < M ? (static_cast<uint32_t>(m0 + 32 * i + r) * K + 16 * h) * XE : kOob;
     const uint32_t ow = n < N ? (static_cast<uint32_t>(n) * K + 16 * h) * 2 : kOob;
+    const float bv = bf16_to_f32(
+        static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(rb, static_cast<uint32_t>(n) * 2, 0, 0)));
     v16f acc[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
     const int nkb = K / BF_KB;
+    uint16_t* xs = reinterpret_cast<uint16_t*>(stage);
     for (int k2 = 0; k2 < nkb; k2 += 2) {
-        v4i xr[2][2][XF32 ? 4 : 2], wr[2][2];
+        // x rows, 64 k: thread t takes 16-byte pieces t, t + 256, ..
+        constexpr int PER_ROW = XF32 ? 16 : 8, PIECES = SK_M * PER_ROW / BF_THR;
+        v4i xr[PIECES], wr[2][2];
 #pragma unroll
-        for (int d = 0; d < 2; ++d) {
-            const uint32_t bad = k2 + d < nkb ? 0u : kOob;  // past K: zeros
-            const uint32_t kb = static_cast<uint32_t>(k2 + d) * BF_KB;
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int q = 0; q < (XF32 ? 4 : 2); ++q)
-                    xr[d][i][q] = __builtin_bit_cast(
-                        v4i, __builtin_amdgcn_raw_buffer_load_b128(rx, ((ox[i] + kb * XE + 16 * q) | (ox[i] & kOob) | bad), 0, 0));
-#pragma unroll
-            for (int q = 0; q < 2; ++q)
-                wr[d][q] = __builtin_bit_cast(
-                    v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, ((ow + kb * 2 + 16 * q) | (ow & kOob) | bad), 0, 0));
+        for (int q = 0; q < PIECES; ++q) {
+            const int row = m0 + (static_cast<int>(threadIdx.x) + BF_THR * q) / PER_ROW;
+            const int k = k2 * BF_KB + (static_cast<int>(threadIdx.x) % PER_ROW) * (16 / XE);
+            xr[q] = __builtin_bit_cast(
+                v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                         rx, row < M && k < K ? (static_cast<uint32_t>(row) * K + k) * XE : kOob, 0, 0));
         }
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
-            v8bf fx[2][2];
+            const uint32_t bad = k2 + d < nkb ? 0u : kOob;  // past K: zeros
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                if constexpr (XF32) {
-                    v4f xv[4];
+            for (int q = 0; q < 2; ++q)
+                wr[d][q] = __builtin_bit_cast(
+                    v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                             rw, ((ow + static_cast<uint32_t>(k2 + d) * BF_KB * 2 + 16 * q) | (ow & kOob) | bad), 0, 0));
+        }
+        if (k2 > 0) __syncthreads();  // every wave has read the previous rows
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) xv[q] = __builtin_bit_cast(v4f, xr[d][i][q]);
-                    f32x16_to_frags(xv, fx[i][0], fx[i][1]);
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) fx[i][q] = __builtin_bit_cast(v8bf, xr[d][i][q]);
-                }
+        for (int q = 0; q < PIECES; ++q) {
+            const int idx = static_cast<int>(threadIdx.x) + BF_THR * q;
+            uint16_t* o = xs + idx / PER_ROW * SK_XP + idx % PER_ROW * (16 / XE);
+            if constexpr (XF32) {
+                const v4f f = __builtin_bit_cast(v4f, xr[q]);
+                *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]));
+            } else {
+                *reinterpret_cast<v4i*>(o) = xr[q];
             }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
 #pragma unroll
             for (int q = 0; q < 2; ++q)
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
-                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[i][q], __builtin_bit_cast(v8bf, wr[d][q]),
-                                                                     acc[i], 0, 0, 0);
-        }
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        *reinterpret_cast<const v8bf*>(xs + (32 * i + r) * SK_XP + 32 * d + 16 * h + 8 * q),
+                        __builtin_bit_cast(v8bf, wr[d][q]), acc[i], 0, 0, 0);
     }
-    const float bv = bf16_to_f32(
-        static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(rb, static_cast<uint32_t>(n) * 2, 0, 0)));
+    __syncthreads();  // the output tile takes x's place
     const bool vec_ok = (N & 3) == 0;
     const int sc = 4 * (threadIdx.x & 31);  // columns this thread stores
     const int sr = threadIdx.x >> 5;        // and its first row
@@ -361,28 +367,27 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __
 #pragma unroll
             for (int e = 0; e < 16; ++e) v[e] = v[e] + prev[e];
         }
-        if (i > 0) __syncthreads();  // the first block's stores have read the stage
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             if (bias != nullptr) v[e] = v[e] + bv;
             if (GELU) v[e] = gelu_tanh(v[e]);
-            stage[(8 * (e >> 2) + 4 * h + (e & 3)) * PITCH + 32 * wave + r] = v[e];
+            stage[(32 * i + 8 * (e >> 2) + 4 * h + (e & 3)) * PITCH + 32 * wave + r] = v[e];
         }
-        __syncthreads();
+    }
+    __syncthreads();
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int row = sr + 8 * q;
-            const v4f t = *reinterpret_cast<const v4f*>(stage + row * PITCH + sc);
-            const uint32_t o = (static_cast<uint32_t>(32 * i + row) * N + n0 + sc) * 4;
-            if (vec_ok) {
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, t), ro, n0 + sc < N ? o : kOob, 0, 0);
-            } else {
+    for (int q = 0; q < SK_M / 8; ++q) {
+        const int row = sr + 8 * q;
+        const v4f t = *reinterpret_cast<const v4f*>(stage + row * PITCH + sc);
+        const uint32_t o = (static_cast<uint32_t>(row) * N + n0 + sc) * 4;
+        if (vec_ok) {
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, t), ro, n0 + sc < N ? o : kOob, 0, 0);
+        } else {
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const float tc = t[c];
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(tc), ro, n0 + sc + c < N ? o + 4 * c : kOob,
-                                                          0, 0);
-                }
+            for (int c = 0; c < 4; ++c) {
+                const float tc = t[c];
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(tc), ro, n0 + sc + c < N ? o + 4 * c : kOob,
+                                                      0, 0);
             }
         }
     }
