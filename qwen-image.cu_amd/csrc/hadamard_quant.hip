@@ -321,6 +321,63 @@ __global__ __launch_bounds__(256) void fwht_quant_blocks_kernel(const InT* x, vo
         }
 }
 
+// The same rows with the NB blocks side by side: 256 NB threads, block
+// tid / 256 by threads tid % 256, the whole row in LDS (52 KB at NB = 3). One
+// block's latency instead of NB in a row, for launches whose rows do not fill
+// the chip anyway. Each value sees the same stages in the same order.
+template <typename InT, RowOut OUT, int NB, bool GELU_IN = false>
+__global__ __launch_bounds__(256 * NB) void fwht_quant_row_at_once_kernel(const InT* x, void* out,
+                                                                          float* __restrict__ scales, float norm) {
+    constexpr int HBS = 4096, K = NB * HBS;
+    extern __shared__ float lds[];
+    float* red = lds + lds_pad(K) + 1;
+    const int row = blockIdx.x;
+    const int tid = threadIdx.x;
+    const int base = (tid >> 8) * HBS + (tid & 255);  // this thread's values after the last sweep: base + 256 i
+    float v[16];
+    load16<InT>(x + static_cast<int64_t>(row) * K + 16 * tid, v);
+    if constexpr (GELU_IN) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = gelu_tanh_fast(v[i]);
+    }
+    butterfly<4>(v);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) lds[lds_pad(16 * tid + i)] = v[i];
+    __syncthreads();
+    float amax = 0.0f;
+    lds_pass<4>(lds, K, 4, false, norm, amax);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = lds[lds_pad(base + (i << 8))];
+    butterfly<4>(v);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        v[i] = v[i] * norm;
+        amax = fmaxf(amax, fabsf(v[i]));
+    }
+    amax = wave_max_dpp(amax);
+    if ((tid & (kWave - 1)) == 0) red[tid / kWave] = amax;
+    __syncthreads();
+    amax = red[0];
+#pragma unroll
+    for (int w = 1; w < 4 * NB; ++w) amax = fmaxf(amax, red[w]);
+    constexpr float QMAX = (OUT == RowOut::Int8) ? 127.0f : 448.0f;
+    if (tid == 0) scales[row] = amax / QMAX;
+    const float inv = (amax > 0.0f) ? QMAX / amax : 0.0f;
+    uint8_t* o = reinterpret_cast<uint8_t*>(out) + static_cast<int64_t>(row) * K + base;
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+        const float q0 = v[i] * inv, q1 = v[i + 1] * inv, q2 = v[i + 2] * inv, q3 = v[i + 3] * inv;
+        uint32_t w;
+        if constexpr (OUT == RowOut::Int8)
+            w = i8x4_rne_sat(q0, q1, q2, q3);
+        else
+            w = e4m3x4(q0, q1, q2, q3);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[(i + c) << 8] = static_cast<uint8_t>(w >> (8 * c));
+    }
+}
+
 // LDS operations of one wave complete in order; this keeps the compiler
 // from moving a read of another lane's value above the write.
 __device__ __forceinline__ void wave_lds_order() {
@@ -1059,26 +1116,60 @@ static hipError_t launch_wave_rows(const Loader& ld, void* out, float* scales, i
     return launch_wave_rows<OUT>(ld, RowDest{out, scales}, M, K, norm, stream);
 }
 
+// Rows of 2-4 Hadamard blocks of 4096 values: up to kAtOnceRows of them with a
+// row's blocks side by side, more with the blocks in turn. K = 12288 fp32, in
+// turn against side by side (us): 1 row 5.8 / 4.4, 269 7.9 / 6.7, 512 8.8 /
+// 7.6, 1024 15.4 / 14.2, 2048 23.8 / 23.4 (HBM-bound from there on, where the
+// smaller buffer keeps more rows in flight).
+constexpr int kAtOnceRows = 1024;
+template <typename InT, RowOut OUT, int NB, bool GELU_IN>
+static hipError_t launch_blocks4096_nb(const InT* x, void* out, float* scales, int M, float norm, hipStream_t stream) {
+    constexpr int K = NB * 4096;
+    if (M <= kAtOnceRows) {
+        const size_t lds = sizeof(float) * (K + K / 16 + 1 + 4 * NB);
+        auto kern = fwht_quant_row_at_once_kernel<InT, OUT, NB, GELU_IN>;
+        if (lds > 64 * 1024) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     static_cast<int>(lds));
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(kern, dim3(M), dim3(256 * NB), lds, stream, x, out, scales, norm);
+    } else {
+        const size_t lds = sizeof(float) * (4096 + 4096 / 16 + 1 + 8);
+        hipLaunchKernelGGL((fwht_quant_blocks_kernel<InT, OUT, NB, GELU_IN>), dim3(M), dim3(256), lds, stream, x, out,
+                           scales, M, K, norm);
+    }
+    return hipGetLastError();
+}
+template <typename InT, RowOut OUT, bool GELU_IN = false>
+static hipError_t launch_blocks4096(const InT* x, void* out, float* scales, int M, int nb, float norm,
+                                    hipStream_t stream) {
+    switch (nb) {
+        case 2: return launch_blocks4096_nb<InT, OUT, 2, GELU_IN>(x, out, scales, M, norm, stream);
+        case 3: return launch_blocks4096_nb<InT, OUT, 3, GELU_IN>(x, out, scales, M, norm, stream);
+        default: return launch_blocks4096_nb<InT, OUT, 4, GELU_IN>(x, out, scales, M, norm, stream);
+    }
+}
+
 template <typename InT, RowOut OUT>
 static hipError_t launch_rows(const InT* x, void* out, float* scales, int M, int K, int hbs,
                               hipStream_t stream) {
     if (M == 0) return hipSuccess;
     const float norm = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(hbs)));
     if constexpr (OUT == RowOut::Int8 || OUT == RowOut::Fp8) {
-        // rows of 1-4 Hadamard blocks of 1024 values: one wave per row
-        if (hbs == 1024 && K % 1024 == 0 && K / 1024 <= 4) {
+        // rows of 1-4 Hadamard blocks of 1024 values: one wave per row; up to
+        // 512 rows do not fill the chip and take a workgroup per row below,
+        // whose waves share the row's latency (3072 bf16, us, wave / workgroup:
+        // 16 rows 4.9 / 4.3, 269 5.4 / 4.5, 512 5.5 / 4.8, 1024 5.9 / 5.7,
+        // 2048 7.5 / 8.2)
+        if (hbs == 1024 && K % 1024 == 0 && K / 1024 <= 4 && M > 512) {
             return launch_wave_rows<OUT>(RowsLoader<InT>{x, K}, out, scales, M, K, norm, stream);
         }
-        // rows of 2-4 Hadamard blocks of 4096 values: block by block
+        // rows of 2-4 Hadamard blocks of 4096 values
         const int nb = K / 4096;
-        if (hbs == 4096 && nb >= 2 && nb <= 4 && nb * 4096 == K) {
-            const size_t lds = sizeof(float) * (4096 + 4096 / 16 + 1 + 8);
-            auto kern = nb == 2 ? fwht_quant_blocks_kernel<InT, OUT, 2>
-                      : nb == 3 ? fwht_quant_blocks_kernel<InT, OUT, 3>
-                                : fwht_quant_blocks_kernel<InT, OUT, 4>;
-            hipLaunchKernelGGL(kern, dim3(M), dim3(256), lds, stream, x, out, scales, M, K, norm);
-            return hipGetLastError();
-        }
+        if (hbs == 4096 && nb >= 2 && nb <= 4 && nb * 4096 == K)
+            return launch_blocks4096<InT, OUT>(x, out, scales, M, nb, norm, stream);
     }
     int chunks = (K + 15) / 16;
     int threads = ((chunks + kWave - 1) / kWave) * kWave;
@@ -1119,17 +1210,10 @@ hipError_t launch_fwht_quant_gelu(const float* x, int M, int K, int hbs, int mod
     if (!fwht_quant_gelu_supported(K, hbs)) return hipErrorNotSupported;
     if (M == 0) return hipSuccess;
     const float norm = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(hbs)));
-    const size_t lds = sizeof(float) * (4096 + 4096 / 16 + 1 + 8);
     const int nb = K / 4096;
-    const bool fp8 = mode == QIMG_QM_FP8_HADAMARD;
-    auto kern = fp8 ? (nb == 2   ? fwht_quant_blocks_kernel<float, RowOut::Fp8, 2, true>
-                       : nb == 3 ? fwht_quant_blocks_kernel<float, RowOut::Fp8, 3, true>
-                                 : fwht_quant_blocks_kernel<float, RowOut::Fp8, 4, true>)
-                    : (nb == 2   ? fwht_quant_blocks_kernel<float, RowOut::Int8, 2, true>
-                       : nb == 3 ? fwht_quant_blocks_kernel<float, RowOut::Int8, 3, true>
-                                 : fwht_quant_blocks_kernel<float, RowOut::Int8, 4, true>);
-    hipLaunchKernelGGL(kern, dim3(M), dim3(256), lds, stream, x, q_out, scales, M, K, norm);
-    return hipGetLastError();
+    return mode == QIMG_QM_FP8_HADAMARD
+               ? launch_blocks4096<float, RowOut::Fp8, true>(x, q_out, scales, M, nb, norm, stream)
+               : launch_blocks4096<float, RowOut::Int8, true>(x, q_out, scales, M, nb, norm, stream);
 }
 
 hipError_t launch_ln_fwht_quant(const float* x, const float* shift, const float* scale, int M, int K, int hbs,
