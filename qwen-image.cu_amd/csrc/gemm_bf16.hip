@@ -398,9 +398,11 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __
 // elements of K of the tile's x and w rows, filled by direct global->LDS DMA
 // of whole lines (1 KB per instruction; the direct fragment loads of
 // gemm_bf16_kernel touch 16 to 64 bytes of each of 32 lines) into a ring of
-// NS stages, NS - 1 in flight. The four waves take 32 elements of K each and
-// compute the whole tile (v_mfma_f32_16x16x32_bf16, w as the A operand), so
-// each operand byte leaves LDS once; x is rounded to bf16 on the fragments.
+// NS stages, NS - 1 in flight. Four waves take 32 elements of K each and compute
+// the whole tile (v_mfma_f32_16x16x32_bf16, w as the A operand), so each operand
+// byte leaves LDS once; tiles of 32 and 64 rows have eight waves, four for each
+// half of the rows (w leaves LDS twice, and a SIMD has a second wave to run
+// while one waits for its fragments). x is rounded to bf16 on the fragments.
 // The partial tiles are summed through LDS in wave order, and the stores run
 // along n. One barrier per stage: stage s has landed in every wave, and every
 // wave is done with stage s - 1, whose slot is refilled right after.
@@ -410,10 +412,11 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_shortk_kernel(const void* __
 // result is rounded to bf16 there, rows of ldo (out is not touched). x has rows
 // of ldx.
 // Measured against gemm_bf16_kernel (us, fp32 x): txt_in 256x3072x3584 48 ->
-// 24, proj_out 4096x64x3072 25 -> 11 (50 MB of x: 4.6 TB/s), norm_out
-// 1x6144x3072 11 -> 7.9 (38 MB of w: 4.8 TB/s); the INT4 down factor
-// 4096x32x3072 (bf16 x) 15.7 -> 6.7. txt_in is bound by the 1.4 MB each of
-// its 192 workgroups reads through its CU's port with 96 KB in flight.
+// 18.4 (23.3 with four waves; 512 rows 44.2 -> 35.8), proj_out 4096x64x3072 25
+// -> 10.9 (50 MB of x: 4.6 TB/s), norm_out 1x6144x3072 11 -> 7.9 (38 MB of w:
+// 4.8 TB/s); the INT4 down factor 4096x32x3072 (bf16 x) 15.7 -> 6.7. txt_in
+// has 192 workgroups that each take 1.4 MB through their CU's port with 96 KB
+// in flight.
 template <bool XF32, int TM, int TN>
 struct BfDma {
     static constexpr int KS = 128;                        // K elements per stage
@@ -422,20 +425,24 @@ struct BfDma {
     static constexpr int XB = TM * XROW, WB = TN * WROW;
     static constexpr int STAGE = XB + WB;
     static constexpr int NS = 144 * 1024 / STAGE < 8 ? 144 * 1024 / STAGE : 8;
-    static constexpr int XI = XB / 4096, WI = WB / 4096;  // DMA instructions per wave and stage
+    static constexpr int MH = TM >= 32 ? 2 : 1;           // waves along the tile's rows
+    static constexpr int NW = 4 * MH, THR = 64 * NW;
+    static constexpr int XI = XB / (1024 * NW), WI = WB / (1024 * NW);  // DMA instructions per wave and stage
     static constexpr int PER = XI + WI;
-    static_assert(XB % 4096 == 0 && WB % 4096 == 0 && NS >= 3 && (NS - 1) * PER <= 63, "stage split over four waves");
+    static_assert(XB % (1024 * NW) == 0 && WB % (1024 * NW) == 0 && NS >= 3 && (NS - 1) * PER <= 63,
+                  "stage split over the waves");
     static_assert(NS * STAGE >= 4 * TM * (TN + 4) * 4, "the partial tiles reuse the ring");
 };
 
 template <bool XF32, int TM, int TN, bool GELU>
-__global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __restrict__ X,
+__global__ __launch_bounds__((BfDma<XF32, TM, TN>::THR)) void gemm_bf16_dma_kernel(const void* __restrict__ X,
                                                                const uint16_t* __restrict__ Wt,
                                                                const uint16_t* __restrict__ bias, float* out,
                                                                uint16_t* out16, int64_t ldx, int64_t ldo, int M,
                                                                int N, int K, int accumulate) {
     using G = BfDma<XF32, TM, TN>;
-    constexpr int NS = G::NS, PER = G::PER, XI = G::XI;
+    constexpr int NS = G::NS, PER = G::PER, XI = G::XI, NW = G::NW;
+    constexpr int WM = TM / G::MH;  // rows of a wave
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * G::STAGE];
 
     const int tiles_m = (M + TM - 1) / TM;
@@ -448,6 +455,8 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __res
     const int n0 = (x_larger ? logical % tiles_n : logical / tiles_m) * TN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ks = wave & 3;           // this wave's 32 elements of a stage's K
+    const int mw = (wave >> 2) * WM;   // and its rows of the tile
 
     // bias of the four columns this thread stores in every row it stores
     const int col = n0 + 4 * (static_cast<int>(threadIdx.x) % (TN / 4));
@@ -455,14 +464,14 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __res
 #pragma unroll
     for (int c = 0; c < 4; ++c) bv[c] = bias != nullptr ? bf16_to_f32(bias[col + c < N ? col + c : N - 1]) : 0.0f;
 
-    // DMA instruction j of this wave fills KB 4 j + wave of the stage (x
+    // DMA instruction j of this wave fills KB NW j + wave of the stage (x
     // rows, then w rows)
     const uint8_t* src[PER];
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         const bool is_x = j < XI;
         const int rb = is_x ? G::XROW : G::WROW;  // bytes per row
-        const int off = (4 * (is_x ? j : j - XI) + wave) * 1024 + lane * 16;
+        const int off = (NW * (is_x ? j : j - XI) + wave) * 1024 + lane * 16;
         const int row = off / rb;
         const int c = ((off % rb) >> 4) ^ (row & 15);
         if (is_x) {
@@ -478,40 +487,40 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __res
 #pragma unroll
         for (int j = 0; j < PER; ++j)
             __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src[j] + static_cast<int64_t>(s) * (j < XI ? G::XROW : G::WROW)),
-                                             (lds_ptr_t)(dst + j * 4096), 16, 0, 1);
+                                             (lds_ptr_t)(dst + j * (NW * 1024)), 16, 0, 1);
     };
 
     const int r = lane & 15;
     const int kq = lane >> 4;
-    v4f acc[TM / 16][TN / 16];
+    v4f acc[WM / 16][TN / 16];
 #pragma unroll
-    for (int i = 0; i < TM / 16; ++i)
+    for (int i = 0; i < WM / 16; ++i)
 #pragma unroll
         for (int j = 0; j < TN / 16; ++j) acc[i][j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-    // lane (row r, kq) of a fragment holds elements 32 wave + 8 kq .. +7
+    // lane (row r, kq) of a fragment holds elements 32 ks + 8 kq .. +7
     auto compute = [&](int slot) {
         const uint8_t* xs = lds + slot * G::STAGE;
         const uint8_t* ws = xs + G::XB;
-        v8bf fx[TM / 16], fw[TN / 16];
+        v8bf fx[WM / 16], fw[TN / 16];
 #pragma unroll
         for (int j = 0; j < TN / 16; ++j)
-            fw[j] = *reinterpret_cast<const v8bf*>(ws + (16 * j + r) * G::WROW + (((4 * wave + kq) ^ r) << 4));
+            fw[j] = *reinterpret_cast<const v8bf*>(ws + (16 * j + r) * G::WROW + (((4 * ks + kq) ^ r) << 4));
 #pragma unroll
-        for (int i = 0; i < TM / 16; ++i) {
-            const uint8_t* row = xs + (16 * i + r) * G::XROW;
+        for (int i = 0; i < WM / 16; ++i) {
+            const uint8_t* row = xs + (mw + 16 * i + r) * G::XROW;
             if constexpr (XF32) {
-                const v4f lo = *reinterpret_cast<const v4f*>(row + (((8 * wave + 2 * kq) ^ r) << 4));
-                const v4f hi = *reinterpret_cast<const v4f*>(row + (((8 * wave + 2 * kq + 1) ^ r) << 4));
+                const v4f lo = *reinterpret_cast<const v4f*>(row + (((8 * ks + 2 * kq) ^ r) << 4));
+                const v4f hi = *reinterpret_cast<const v4f*>(row + (((8 * ks + 2 * kq + 1) ^ r) << 4));
                 fx[i] = __builtin_bit_cast(v8bf, (v4i){static_cast<int>(pack_bf16x2(lo[0], lo[1])),
                                                        static_cast<int>(pack_bf16x2(lo[2], lo[3])),
                                                        static_cast<int>(pack_bf16x2(hi[0], hi[1])),
                                                        static_cast<int>(pack_bf16x2(hi[2], hi[3]))});
             } else {
-                fx[i] = *reinterpret_cast<const v8bf*>(row + (((4 * wave + kq) ^ r) << 4));
+                fx[i] = *reinterpret_cast<const v8bf*>(row + (((4 * ks + kq) ^ r) << 4));
             }
         }
 #pragma unroll
-        for (int i = 0; i < TM / 16; ++i)
+        for (int i = 0; i < WM / 16; ++i)
 #pragma unroll
             for (int j = 0; j < TN / 16; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[j], fx[i], acc[i][j], 0, 0, 0);
@@ -547,15 +556,15 @@ __global__ __launch_bounds__(BF_THR) void gemm_bf16_dma_kernel(const void* __res
     constexpr int PITCH = TN + 4;
     float* red = reinterpret_cast<float*>(lds);
 #pragma unroll
-    for (int i = 0; i < TM / 16; ++i)
+    for (int i = 0; i < WM / 16; ++i)
 #pragma unroll
         for (int j = 0; j < TN / 16; ++j)
-            *reinterpret_cast<v4f*>(red + (wave * TM + 16 * i + r) * PITCH + 16 * j + 4 * kq) = acc[i][j];
+            *reinterpret_cast<v4f*>(red + (ks * TM + mw + 16 * i + r) * PITCH + 16 * j + 4 * kq) = acc[i][j];
     __syncthreads();
     const bool vec_ok = (N & 3) == 0;
 #pragma unroll
-    for (int q = 0; q < (TM * TN / 4 + BF_THR - 1) / BF_THR; ++q) {
-        const int idx = static_cast<int>(threadIdx.x) + BF_THR * q;
+    for (int q = 0; q < (TM * TN / 4 + G::THR - 1) / G::THR; ++q) {
+        const int idx = static_cast<int>(threadIdx.x) + G::THR * q;
         const int row = idx / (TN / 4);
         const int m = m0 + row;
         if (row >= TM || m >= M || col >= N) continue;
@@ -646,10 +655,10 @@ hipError_t launch_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N
                            uint16_t* out16, int64_t ldx, int64_t ldo, int gelu, int accumulate, hipStream_t stream) {
     const int tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     if (gelu)
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, true>), dim3(tiles), dim3(BF_THR), 0, stream, x, w,
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, true>), dim3(tiles), dim3((BfDma<XF32, TM, TN>::THR)), 0, stream, x, w,
                            bias, out, out16, ldx, ldo, M, N, K, accumulate);
     else
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, false>), dim3(tiles), dim3(BF_THR), 0, stream, x, w,
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, false>), dim3(tiles), dim3((BfDma<XF32, TM, TN>::THR)), 0, stream, x, w,
                            bias, out, out16, ldx, ldo, M, N, K, accumulate);
     return hipGetLastError();
 }
