@@ -1167,11 +1167,15 @@ static hipError_t launch_rows(const InT* x, void* out, float* scales, int M, int
     const float norm = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(hbs)));
     if constexpr (OUT == RowOut::Int8 || OUT == RowOut::Fp8) {
         // rows of 1-4 Hadamard blocks of 1024 values: one wave per row; up to
-        // 512 rows do not fill the chip and take a workgroup per row below,
-        // whose waves share the row's latency (3072 bf16, us, wave / workgroup:
-        // 16 rows 4.9 / 4.3, 269 5.4 / 4.5, 512 5.5 / 4.8, 1024 5.9 / 5.7,
-        // 2048 7.5 / 8.2)
-        if (hbs == 1024 && K % 1024 == 0 && K / 1024 <= 4 && M > 512) {
+        // 512 rows (3 blocks of fp32: 384) of 3 or 4 blocks do not fill the
+        // chip and take a workgroup per row below, whose waves share the row's
+        // latency (3072 bf16, us, wave / workgroup: 16 rows 4.7 / 4.0, 269 5.0
+        // / 4.4, 512 5.2 / 4.6, 1024 5.9 / 5.7, 2048 7.5 / 8.2; fp32 to e4m3
+        // 269 4.57 / 4.51, 512 4.66 / 4.82; 4096 bf16: 269 rows 6.4 / 4.6). One
+        // or two blocks are less work than the workgroup's barriers cost (1024:
+        // 1 row 2.4 / 3.2, 269 3.0 / 3.7; 2048: 3.3 / 3.6, 4.0 / 4.1).
+        const int few = sizeof(InT) == 4 && K == 3072 ? 384 : 512;
+        if (hbs == 1024 && K % 1024 == 0 && K / 1024 <= 4 && (M > few || K / 1024 <= 2)) {
             return launch_wave_rows<OUT>(RowsLoader<InT>{x, K}, out, scales, M, K, norm, stream);
         }
         // rows of 2-4 Hadamard blocks of 4096 values

@@ -249,7 +249,7 @@ def test_quant_repeatable_and_empty(qimg):
     assert e[0].shape == (0, 3072)
 
 
-@pytest.mark.parametrize("K,hbs", [(3072, 1024), (4096, 1024), (8192, 4096), (12288, 4096), (16384, 4096)])
+@pytest.mark.parametrize("K,hbs", [(2048, 1024), (3072, 1024), (4096, 1024), (8192, 4096), (12288, 4096), (16384, 4096)])
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_quant_rows_do_not_depend_on_their_number(qimg, K, hbs, fp8, bf16):
@@ -262,6 +262,6 @@ def test_quant_rows_do_not_depend_on_their_number(qimg, K, hbs, fp8, bf16):
     x = x.bfloat16() if bf16 else x
     mode = qimg.FP8_HADAMARD if fp8 else qimg.INT8_HADAMARD
     ref_q, ref_s = qimg.quantize_activation_hadamard(x, hbs, mode)[:2]
-    for M in (1, 5, 512, 513, 1024, 1025):
+    for M in (1, 5, 384, 385, 512, 513, 1024, 1025):
         q, s = qimg.quantize_activation_hadamard(x[:M], hbs, mode)[:2]
         assert torch.equal(q.view(torch.uint8), ref_q[:M].view(torch.uint8)) and torch.equal(s, ref_s[:M]), M
