@@ -15,6 +15,8 @@
 // rescaled and accumulated in fp32 in the reference's operation order,
 // acc = acc + ((float)d * as[g,m]) * ws[g,n] (w4a4_gemm_regdirect_kernel,
 // cuda_kernels.cu:4206-4212), so the result is the same for every tiling.
+#include <algorithm>
+
 #include "qimg_device.h"
 #include "qimg_internal.h"
 
@@ -34,31 +36,55 @@ __device__ __forceinline__ float int4_code(int n, int nf4, int signed_int4) {
     return static_cast<float>(signed_int4 ? nib_signed(n) : n - 8);
 }
 
+// The row passes below take `per` threads a row. Short rows share a workgroup
+// of SHORT_THR threads, rpw of them side by side; others are nb parts of THR
+// threads. Workgroups stride over the rows. (One kernel for both, and a grid of
+// parts by rows, cost the long rows 0.2 us.)
+constexpr int ROW_THR = 128, SHORT_THR = 256;
+struct RowThread {
+    int row, sub, col, step;  // the thread's first row (its sub-th of the workgroup's), its place in it, rows to the next
+    bool live;                // false: past the last of the rpw rows
+};
+template <bool SHORT, int THR>
+__device__ __forceinline__ RowThread row_thread(int per, int nb) {
+    const int tid = static_cast<int>(threadIdx.x);
+    if constexpr (SHORT) {
+        // quotients of numbers up to 256, at least 1/512 from the next integer
+        const float inv = __builtin_amdgcn_rcpf(static_cast<float>(per));
+        const int rpw = static_cast<int>((SHORT_THR + 0.5f) * inv);
+        const int sub = static_cast<int>((static_cast<float>(tid) + 0.5f) * inv);
+        return {static_cast<int>(blockIdx.x) * rpw + sub, sub, tid - sub * per, static_cast<int>(gridDim.x) * rpw,
+                sub < rpw};
+    }
+    return {static_cast<int>(blockIdx.x / nb), 0, static_cast<int>(blockIdx.x % nb) * THR + tid,
+            static_cast<int>(gridDim.x / nb), true};
+}
+
 // dequantize_int4_to_bf16_kernel (cuda_kernels.cu:2876-2917): one thread per
-// 4 packed bytes (8 columns, one 16-byte bf16 store), K % 8 == 0, nb blocks of
-// threads along a row and a stride of gridDim.x / nb rows. Bound by writing
-// the output; the next row's words are loaded before this one's are used. With
-// pad > 0 a row of out is K + pad long, columns K .. K + r taken from up [N, r]
-// and the rest zero. A byte's two code values come from an LDS table (grid lookups
-// from constant memory and 64-bit divisions per thread had made it 13.5 us at
-// 3072 x 3072, 1.7 TB/s; now 9.4 us).
-constexpr int ROW_THR = 128;
-__global__ __launch_bounds__(ROW_THR) void dequant_int4_bf16_kernel(const uint8_t* __restrict__ qw,
-                                                                    const float* __restrict__ scales,
-                                                                    uint16_t* __restrict__ out, int N, int K, int gs,
-                                                                    int nf4, int scales_gn, int signed_int4,
-                                                                    const uint16_t* __restrict__ up, int r, int pad,
-                                                                    int nb) {
+// 4 packed bytes (8 columns, one 16-byte bf16 store), K % 8 == 0. Bound by
+// writing the output; the next row's words are loaded before this one's are
+// used. With pad > 0 a row of out is K + pad long, columns K .. K + r taken
+// from up [N, r] and the rest zero. A byte's two code values come from an LDS
+// table (grid lookups from constant memory and 64-bit divisions per thread had
+// made it 13.5 us at 3072 x 3072, 1.7 TB/s; now 9.4 us).
+template <bool SHORT>
+__global__ __launch_bounds__(SHORT ? SHORT_THR : ROW_THR) void dequant_int4_bf16_kernel(const uint8_t* __restrict__ qw,
+                                                                const float* __restrict__ scales,
+                                                                uint16_t* __restrict__ out, int N, int K, int gs,
+                                                                int nf4, int scales_gn, int signed_int4,
+                                                                const uint16_t* __restrict__ up, int r, int pad, int nb) {
     __shared__ float2 table[256];
-    for (int i = threadIdx.x; i < 256; i += ROW_THR)
+    for (int i = threadIdx.x; i < 256; i += SHORT ? SHORT_THR : ROW_THR)
         table[i] = make_float2(int4_code(i & 15, nf4, signed_int4), int4_code(i >> 4, nf4, signed_int4));
     __syncthreads();
     const int G = K / gs;
-    const int word = (blockIdx.x % nb) * ROW_THR + threadIdx.x;
-    const int c0 = word * 8;
     const int64_t ldo = K + pad;
-    const int stride = gridDim.x / nb;
-    int row = blockIdx.x / nb;
+    const RowThread t = row_thread<SHORT, ROW_THR>((K + pad) / 8, nb);
+    if (!t.live) return;
+    const int word = t.col;
+    const int c0 = word * 8;
+    const int stride = t.step;
+    int row = t.row;
     if (c0 >= K) {
         if (c0 >= ldo) return;
         for (; row < N; row += stride) {
@@ -93,10 +119,10 @@ __global__ __launch_bounds__(ROW_THR) void dequant_int4_bf16_kernel(const uint8_
         u32x4 o;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            const float2 t = table[(w >> (8 * p)) & 0xff];
+            const float2 v = table[(w >> (8 * p)) & 0xff];
             const float s0 = one ? s : scale(row, (c0 + 2 * p) / gs);
             const float s1 = one ? s : scale(row, (c0 + 2 * p + 1) / gs);
-            o[p] = pack_bf16x2(t.x * s0, t.y * s1);
+            o[p] = pack_bf16x2(v.x * s0, v.y * s1);
         }
         reinterpret_cast<u32x4*>(out + row * ldo)[word] = o;
     }
@@ -150,66 +176,82 @@ __global__ __launch_bounds__(256) void quant_int4_weight_kernel(const float* __r
 
 // Activation INT4 quant (quantize_activation_int4_kernel, cuda_kernels.cu:
 // 3575-3636; with a smooth divide and a bf16 copy, fused_smooth_bf16_quant_
-// kernel, :3650-3705). A thread owns 8 columns of a row (32 bytes in, 16 and 4
-// out), nb blocks of threads along a row and a stride of gridDim.x / nb rows;
-// a group of gs columns is gs/8 consecutive lanes of one wave (gs = 32, 64 or
-// 128), reduced with lane exchanges. scales [G, M]. Bound by HBM, the IEEE
-// divisions next; with 2 columns a thread, a 64-bit division per thread and
-// 1-byte stores 4352 x 3072 took 33.9 us (2.5 TB/s), now 20.2 us (4.3 TB/s).
-template <int GS>
-__global__ __launch_bounds__(ROW_THR) void quant_act_int4_kernel(const float* __restrict__ x,
+// kernel, :3650-3705). A thread owns V columns of a row; a group of gs
+// columns is gs/V consecutive lanes of one wave (gs = 32, 64 or 128), reduced
+// with lane exchanges. scales [G, M]. Bound by HBM, the IEEE divisions next:
+// 8 columns (32 bytes in, 16 and 4 out) took 4352 x 3072 from 33.9 us (2.5
+// TB/s; 2 columns, a 64-bit division per thread and 1-byte stores) to 20.2 us
+// (4.3 TB/s). A few rows do not fill the chip, and a thread's chain of 8 is
+// what counts: they have 2 columns a thread (16 x 3072 2.37 -> 2.19 us).
+template <int GS, int V, bool SHORT>
+__global__ __launch_bounds__(SHORT || V == 2 ? 256 : ROW_THR) void quant_act_int4_kernel(const float* __restrict__ x,
                                                                  const float* __restrict__ smooth,
                                                                  uint16_t* __restrict__ bf16_out,
                                                                  uint8_t* __restrict__ packed,
                                                                  float* __restrict__ scales, int M, int K, int nb) {
-    const int c = ((blockIdx.x % nb) * ROW_THR + static_cast<int>(threadIdx.x)) * 8;
-    // every lane takes part in the exchanges; lanes past the row hold zeros
-    const bool live = c < K;
-    float sm[8];
-    if (smooth != nullptr && live) {
+    typedef float vec __attribute__((ext_vector_type(V < 4 ? V : 4)));
+    constexpr int E = V < 4 ? V : 4, H = V / E;  // elements per load, loads
+    const RowThread t = row_thread<SHORT, V == 2 ? 256 : ROW_THR>(K / V, nb);
+    const int c = t.col * V;
+    // every lane takes part in the exchanges; lanes past the row or the last
+    // row hold zeros
+    const bool in_row = c < K && t.live;
+    float sm[V];
+    if (smooth != nullptr && in_row) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const v4f t = reinterpret_cast<const v4f*>(smooth + c)[h];
+        for (int h = 0; h < H; ++h) {
+            const vec u = reinterpret_cast<const vec*>(smooth + c)[h];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sm[4 * h + e] = t[e];
+            for (int e = 0; e < E; ++e) sm[E * h + e] = u[e];
         }
     }
-    for (int m = blockIdx.x / nb; m < M; m += gridDim.x / nb) {
-        float v[8] = {};
+    // (m0: the workgroup's first row, for whole waves)
+    for (int m0 = SHORT ? blockIdx.x * (t.step / gridDim.x) : t.row; m0 < M; m0 += t.step) {
+        const int m = SHORT ? m0 + t.sub : m0;
+        const bool live = SHORT ? in_row && m < M : in_row;
+        float v[V] = {};
         if (live) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const v4f t = reinterpret_cast<const v4f*>(x + static_cast<int64_t>(m) * K + c)[h];
+            for (int h = 0; h < H; ++h) {
+                const vec u = reinterpret_cast<const vec*>(x + static_cast<int64_t>(m) * K + c)[h];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[4 * h + e] = t[e];
+                for (int e = 0; e < E; ++e) v[E * h + e] = u[e];
             }
             if (smooth != nullptr) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = v[e] / sm[e];
+                for (int e = 0; e < V; ++e) v[e] = v[e] / sm[e];
             }
             if (bf16_out != nullptr) {
-                u32x4 o;
+                uint16_t* o = bf16_out + static_cast<int64_t>(m) * K + c;
+                uint32_t w[V / 2];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(v[2 * e], v[2 * e + 1]);
-                *reinterpret_cast<u32x4*>(bf16_out + static_cast<int64_t>(m) * K + c) = o;
+                for (int e = 0; e < V / 2; ++e) w[e] = pack_bf16x2(v[2 * e], v[2 * e + 1]);
+                if constexpr (V == 8)
+                    *reinterpret_cast<u32x4*>(o) = (u32x4){w[0], w[1], w[2], w[3]};
+                else
+                    *reinterpret_cast<uint32_t*>(o) = w[0];
             }
         }
         float amax = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
+        for (int e = 0; e < V; ++e) amax = fmaxf(amax, fabsf(v[e]));
 #pragma unroll
-        for (int off = 1; off < GS / 8; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
+        for (int off = 1; off < GS / V; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
         if (!live) continue;
         if ((c % GS) == 0) scales[static_cast<int64_t>(c / GS) * M + m] = amax / 7.0f;
         const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
         uint32_t w = 0;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < V; ++e) {
             int q = static_cast<int>(roundf(v[e] * inv));
             q = q < -7 ? -7 : (q > 7 ? 7 : q);
             w |= static_cast<uint32_t>(q & 0xF) << (4 * e);
         }
-        *reinterpret_cast<uint32_t*>(packed + static_cast<int64_t>(m) * (K / 2) + c / 2) = w;
+        uint8_t* o = packed + static_cast<int64_t>(m) * (K / 2) + c / 2;
+        if constexpr (V == 8)
+            *reinterpret_cast<uint32_t*>(o) = w;
+        else
+            *o = static_cast<uint8_t>(w);
     }
 }
 
@@ -735,8 +777,20 @@ int grid_for(int64_t n, int per_block = 256) {
     return static_cast<int>(b < 65536 ? (b > 0 ? b : 1) : 65536);
 }
 
-// Workgroups of ROW_THR threads of 8 columns along a row.
-int row_blocks(int K) { return (K / 8 + ROW_THR - 1) / ROW_THR; }
+// Parts of a row and grid of a row pass with `per` threads a row, at most
+// `most` workgroups (below 2^24: a launch holds fewer than 2^32 threads).
+struct RowGrid {
+    int nb;
+    unsigned blocks;
+};
+RowGrid row_grid(int rows, int per, bool is_short, int threads, int most) {
+    if (is_short) {
+        const int rpw = SHORT_THR / per, parts = (rows - 1) / rpw + 1;
+        return {1, static_cast<unsigned>(std::min(parts, most))};
+    }
+    const int nb = (per + threads - 1) / threads;
+    return {nb, static_cast<unsigned>(nb) * std::min(rows, nb < most ? most / nb : 1)};
+}
 
 }  // namespace
 
@@ -750,11 +804,19 @@ hipError_t launch_dequant_int4_bf16_ext(const uint8_t* qw, const float* scales, 
                                         hipStream_t stream) {
     if (N == 0 || K == 0) return hipSuccess;
     if (K % 8 != 0 || gs <= 0 || K % gs != 0 || pad < r || pad % 8 != 0) return hipErrorInvalidValue;
-    // about 4096 workgroups: each loads its table for a few rows
-    const int nb = row_blocks(K + pad);
-    const int rows = nb < 4096 ? 4096 / nb : 1;
-    hipLaunchKernelGGL(dequant_int4_bf16_kernel, dim3(static_cast<unsigned>(nb) * (N < rows ? N : rows)), dim3(ROW_THR),
-                       0, stream, qw, scales, out, N, K, gs, nf4, scales_gn, signed_int4, up, r, pad, nb);
+    // at most 4096 workgroups: each loads its table for a few rows
+    const int per = (K + pad) / 8;
+    // short: rows that would leave more than half of ROW_THR idle (us, one row
+    // a workgroup / side by side: 50000 x 8 8.7 / 2.6, 12288 x 64 5.3 / 2.8,
+    // 3072 x 256 4.0 / 2.8; 12288 x 512 6.5 / 7.4)
+    const bool is_short = per < 64;
+    const RowGrid g = row_grid(N, per, is_short, ROW_THR, 4096);
+    if (is_short)
+        hipLaunchKernelGGL(dequant_int4_bf16_kernel<true>, dim3(g.blocks), dim3(SHORT_THR), 0, stream, qw, scales, out,
+                           N, K, gs, nf4, scales_gn, signed_int4, up, r, pad, g.nb);
+    else
+        hipLaunchKernelGGL(dequant_int4_bf16_kernel<false>, dim3(g.blocks), dim3(ROW_THR), 0, stream, qw, scales, out,
+                           N, K, gs, nf4, scales_gn, signed_int4, up, r, pad, g.nb);
     return hipGetLastError();
 }
 
@@ -772,31 +834,35 @@ hipError_t launch_quant_int4_weight(const float* r, uint8_t* qw, float* scales, 
     return hipGetLastError();
 }
 
+template <int GS, int V>
+static void run_quant_act(const float* x, const float* smooth, uint16_t* bf16_out, uint8_t* packed, float* scales,
+                          int M, int K, hipStream_t stream) {
+    constexpr int THR = V == 2 ? 256 : ROW_THR;
+    // 8 columns: as in the dequantization (30000 x 64 13.0 -> 2.9 us, 4352 x 128
+    // 3.8 -> 2.5)
+    const bool is_short = K / V < (V == 2 ? SHORT_THR : 64);
+    const RowGrid g = row_grid(M, K / V, is_short, THR, 1 << 23);
+    if (is_short)
+        hipLaunchKernelGGL((quant_act_int4_kernel<GS, V, true>), dim3(g.blocks), dim3(SHORT_THR), 0, stream, x, smooth,
+                           bf16_out, packed, scales, M, K, g.nb);
+    else
+        hipLaunchKernelGGL((quant_act_int4_kernel<GS, V, false>), dim3(g.blocks), dim3(THR), 0, stream, x, smooth,
+                           bf16_out, packed, scales, M, K, g.nb);
+}
+
 hipError_t launch_quant_act_int4(const float* x, const float* smooth, uint16_t* bf16_out, uint8_t* packed,
                                  float* scales, int M, int K, int gs, hipStream_t stream) {
     if (M == 0 || K == 0) return hipSuccess;
-    if (K % gs != 0) return hipErrorInvalidValue;
-    // one workgroup per row part, up to 2^23 of them (a launch holds fewer
-    // than 2^32 threads); past that they stride over the rows
-    const int nb = row_blocks(K);
-    const int rows = nb < (1 << 23) ? (1 << 23) / nb : 1;
-    const dim3 grid(static_cast<unsigned>(nb) * (M < rows ? M : rows));
-    switch (gs) {
-        case 32:
-            hipLaunchKernelGGL(quant_act_int4_kernel<32>, grid, dim3(ROW_THR), 0, stream, x, smooth, bf16_out, packed,
-                               scales, M, K, nb);
-            break;
-        case 64:
-            hipLaunchKernelGGL(quant_act_int4_kernel<64>, grid, dim3(ROW_THR), 0, stream, x, smooth, bf16_out, packed,
-                               scales, M, K, nb);
-            break;
-        case 128:
-            hipLaunchKernelGGL(quant_act_int4_kernel<128>, grid, dim3(ROW_THR), 0, stream, x, smooth, bf16_out,
-                               packed, scales, M, K, nb);
-            break;
-        default:
-            return hipErrorInvalidValue;
-    }
+    if ((gs != 32 && gs != 64 && gs != 128) || K % gs != 0) return hipErrorInvalidValue;
+    // us, 2 / 8 columns a thread: 16 x 3072 2.19 / 2.37, 128 x 3072 2.5 / 2.6,
+    // 128 x 128 2.1 / 2.4; past the line 192 x 3072 2.8 / 2.7, 512 x 1024 2.8 /
+    // 2.7; rows that are no whole workgroups of 8 columns 128 x 1056 2.5 / 2.3,
+    // 128 x 1536 2.5 / 2.25
+    const bool few = static_cast<int64_t>(M) * K <= 3 << 17 && (K < 512 || K % 1024 == 0);
+    auto* run = few
+                    ? (gs == 32 ? run_quant_act<32, 2> : gs == 64 ? run_quant_act<64, 2> : run_quant_act<128, 2>)
+                    : (gs == 32 ? run_quant_act<32, 8> : gs == 64 ? run_quant_act<64, 8> : run_quant_act<128, 8>);
+    run(x, smooth, bf16_out, packed, scales, M, K, stream);
     return hipGetLastError();
 }
 

@@ -362,17 +362,24 @@ def test_linear_int4_rejects_bad_arguments(qimg):
 
 
 @pytest.mark.parametrize("M,K,gs,smooth", [(5, 32, 32, True), (3, 1056, 32, True), (2, 1152, 128, False),
-                                           (131, 1024, 64, True), (1, 2112, 64, True)])
+                                           (131, 1024, 64, True), (1, 2112, 64, True), (257, 96, 32, False),
+                                           (384, 1024, 64, True), (385, 1024, 64, True), (20003, 32, 32, True),
+                                           (9001, 64, 64, False), (4101, 192, 64, True), (701, 1152, 128, True),
+                                           (1301, 1056, 32, False)])
 def test_quantize_activation_int4_row_parts_bit_exact(qimg, oracle, M, K, gs, smooth):
-    """Rows around the 1024 columns a workgroup of the quantizer takes."""
+    """Rows around the columns a workgroup of the quantizer takes and several
+    short rows to a workgroup, on both sides of its switch from 2 to 8 columns
+    a thread (3 * 2^17 values)."""
     test_quantize_activation_int4_bit_exact(qimg, oracle, M, K, gs, smooth)
 
 
-@pytest.mark.parametrize("N,K,gs", [(3, 1032, 8), (2, 1024, 64), (1400, 1040, 16), (5, 96, 6), (4097, 8, 8)])
+@pytest.mark.parametrize("N,K,gs", [(3, 1032, 8), (2, 1024, 64), (1400, 1040, 16), (5, 96, 6), (4097, 8, 8),
+                                    (50001, 8, 8), (12289, 64, 64), (777, 96, 6), (4100, 520, 8), (5001, 1032, 8),
+                                    (5000, 1544, 8)])
 @pytest.mark.parametrize("form", ["nf4", "linear", "signed_gn"])
 def test_dequant_int4_row_parts_bit_exact(qimg, oracle, N, K, gs, form):
-    """Rows around 1024 columns, groups that end inside 8 columns, and more
-    rows than one pass of the grid."""
+    """Rows around 1024 columns, groups that end inside 8 columns, short rows
+    side by side in a workgroup, and more rows than one pass of the grid."""
     test_dequant_int4_bit_exact(qimg, oracle, N, K, gs, form)
 
 
