@@ -845,8 +845,10 @@ __global__ __launch_bounds__(256) void smooth_fwht_rows_kernel(const float* x, c
     }
     const int64_t base = static_cast<int64_t>(row) * K;
     int lo = 0;
-    if ((K & 15) == 0 && hbs_log2 > 4) {
+    if ((K & 15) == 0 && hbs_log2 > 4 && K >= 256) {
         // 16 values a thread: the first four stages run on its registers
+        // (short rows leave it too few threads: 4352 x 96, h 32, 4.2 us with
+        // a value a thread, 4.8 so; 1024 x 256, h 256, 4.1 and 3.4)
         for (int c = threadIdx.x; c < (K >> 4); c += blockDim.x) {
             float v[16];
             smooth_chunk(x + base, smooth, xs != nullptr ? xs + base : nullptr, c, v);

@@ -427,3 +427,20 @@ def test_linear_w4a16_low_rank_columns(qimg, oracle, M, N, K, r, hbs, smooth, nf
     assert float((got - sep).abs().max()) <= bound
     with pytest.raises(qimg.QimgError):
         qimg.linear_forward_int4(x, w, scratch=torch.empty(least - 256, dtype=torch.uint8, device=DEV))
+
+
+@pytest.mark.parametrize("M,K,hbs", [(3, 32, 32), (5, 96, 32), (4, 128, 128), (7, 240, 16), (6, 240, 8), (2, 256, 32),
+                                     (3, 272, 16), (2, 512, 512), (2, 1056, 32), (3, 4096, 4096), (2, 12288, 4096)])
+@pytest.mark.parametrize("smooth", [False, True])
+def test_smooth_hadamard_bit_exact(qimg, oracle, M, K, hbs, smooth):
+    """Rows on both sides of 256 columns, where the first stages move to a
+    thread's registers, and in place."""
+    rng = np.random.default_rng(K + hbs)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    sm = np.exp(0.3 * rng.standard_normal(K)).astype(np.float32) if smooth else None
+    ref = oracle.fwht_rows(x / sm if smooth else x, hbs)
+    xd = _f32(x)
+    got = qimg.smooth_hadamard(xd, _f32(sm) if smooth else None, hbs)
+    np.testing.assert_array_equal(got.cpu().numpy(), ref)
+    qimg.smooth_hadamard(xd, _f32(sm) if smooth else None, hbs, out=xd)
+    np.testing.assert_array_equal(xd.cpu().numpy(), ref)
