@@ -678,6 +678,60 @@ __global__ __launch_bounds__(AWQ_THR, 5) void awq_gemv_kernel(const float* __res
     out[so] = acc;
 }
 
+// The same with one wave per 64 channels doing all of it, the next group's
+// eight words loaded while this one is summed: for a few groups, where the
+// ring's prologue costs more than the chain, and for more channels than the
+// ring's workgroups can be on the chip at once (awq_short has the line).
+__global__ __launch_bounds__(64) void awq_gemv_short_kernel(const float* __restrict__ x, const int32_t* __restrict__ qw,
+                                                            const uint16_t* __restrict__ wscales,
+                                                            const uint16_t* __restrict__ wzeros,
+                                                            const uint16_t* __restrict__ bias, float* __restrict__ out,
+                                                            int OC, int IC, int ncomp) {
+    extern __shared__ float s_x[];
+    for (int i = threadIdx.x; i < IC; i += blockDim.x) s_x[i] = x[i];
+    __syncthreads();
+    const int nk_raw = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = nk_raw < OC;
+    const int nk = live ? nk_raw : OC - 1;
+    const int G = IC / 64;
+    auto load = [&](int g, uint32_t* p, uint16_t& s, uint16_t& z) {
+#pragma unroll
+        for (int io = 0; io < 8; ++io) p[io] = static_cast<uint32_t>(qw[static_cast<int64_t>(g * 8 + io) * OC + nk]);
+        s = wscales[static_cast<int64_t>(g) * OC + nk];
+        z = wzeros[static_cast<int64_t>(g) * OC + nk];
+    };
+    uint32_t p[8], pn[8];
+    uint16_t s16, z16, sn16 = 0, zn16 = 0;
+    load(0, p, s16, z16);
+    float acc = 0.0f;
+    for (int g = 0; g < G; ++g) {
+        if (g + 1 < G) load(g + 1, pn, sn16, zn16);
+        const float s = bf16_to_f32(s16);
+        const float z = bf16_to_f32(z16);
+        const v4f* xv = reinterpret_cast<const v4f*>(s_x + g * 64);
+#pragma unroll
+        for (int io = 0; io < 8; ++io) {
+            const v4f x0 = xv[2 * io], x1 = xv[2 * io + 1];
+            const float xs[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+#pragma clang fp contract(off)
+                const float w = static_cast<float>((p[io] >> (4 * k)) & 0xF) * s + z;
+                acc = acc + w * xs[k];
+            }
+        }
+#pragma unroll
+        for (int io = 0; io < 8; ++io) p[io] = pn[io];
+        s16 = sn16;
+        z16 = zn16;
+    }
+    if (!live) return;
+    const int dim = OC / ncomp;
+    const int so = (nk % ncomp) * dim + nk / ncomp;
+    if (bias != nullptr) acc = acc + bf16_to_f32(bias[so]);
+    out[so] = acc;
+}
+
 // ---- nunchaku layouts ----------------------------------------------------
 // MMA-swizzled nibble and scale addresses (cuda_kernels.cu:2945-2973).
 __device__ __forceinline__ int nk_nibble(const uint8_t* q, int K, int row, int col) {
@@ -908,11 +962,27 @@ hipError_t launch_awq_dequant(const int32_t* qw, const uint16_t* wscales, const 
     return hipGetLastError();
 }
 
+// Which AWQ kernel, by how often over the ring's workgroups fill the chip (two
+// fit a CU up to 4096 inputs, later one). us, awq_gemv_short_kernel / the ring:
+// up to once, 18432 channels of 128 inputs 4.1 / 5.1, of 192 5.4 / 5.3, of 256
+// 6.4 / 5.3; to 1.5 times, 36864 of 320 7.8 / 8.1, of 384 9.0 / 8.1; to 2.5
+// times, 64000 of 768 15.5 / 19.1, 73728 of 1024 27.4 / 22.6; from there 98304
+// of 896 24 / 28, of 3072 75 / 77, 147456 of 2048 65 / 74.
+static bool awq_short(int OC, int IC) {
+    const int at_once = 256 * (IC <= 4096 ? 2 : 1), wgs = (OC + 63) / 64;
+    return 2 * wgs > 5 * at_once || IC <= 64 * (wgs <= at_once ? 2 : 2 * wgs <= 3 * at_once ? 5 : 12);
+}
+
 hipError_t launch_awq_gemv(const float* x, const int32_t* qw_rep, const uint16_t* wscales, const uint16_t* wzeros,
                            const uint16_t* bias, float* out, int OC, int IC, int gs, int ncomp, hipStream_t stream) {
     if (OC == 0) return hipSuccess;
     // the reference's GEMV reads 8 words (64 inputs) per group
     if (gs != 64 || IC % 64 != 0 || ncomp <= 0 || OC % ncomp != 0 || IC > 16384) return hipErrorInvalidValue;
+    if (awq_short(OC, IC)) {
+        hipLaunchKernelGGL(awq_gemv_short_kernel, dim3((OC + 63) / 64), dim3(64), IC * sizeof(float), stream, x, qw_rep,
+                           wscales, wzeros, bias, out, OC, IC, ncomp);
+        return hipGetLastError();
+    }
     const int lds = AWQ_RING * 16 + IC * 4;
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(awq_gemv_kernel),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);

@@ -158,10 +158,13 @@ def test_awq_paths_bit_exact(qimg, oracle):
 
 
 @pytest.mark.parametrize("OC,IC,nc,bias", [(68, 64, 1, True), (60, 192, 6, False), (64, 576, 2, True),
-                                           (132, 640, 3, True), (72, 16384, 6, True)])
+                                           (132, 640, 3, True), (72, 16384, 6, True), (200, 128, 2, False),
+                                           (32832, 320, 6, True), (32772, 384, 1, False), (49220, 768, 1, True),
+                                           (49220, 832, 2, True), (81984, 832, 1, True), (260, 192, 4, True)])
 def test_awq_gemv_edges_bit_exact(qimg, oracle, OC, IC, nc, bias):
     """Channels past a workgroup's 64, one group, an odd number of groups (a
-    half-filled last stage), fewer stages than are in flight, the longest row."""
+    half-filled last stage), fewer stages than are in flight, the longest row,
+    and both sides of the rule for few groups or many channels."""
     rng = np.random.default_rng(OC + IC)
     rep = rng.integers(-2 ** 31, 2 ** 31, (IC // 8, OC), dtype=np.int64).astype(np.int32)
     ws = oracle.bf16_bits_from_f32(rng.uniform(0.001, 0.02, (IC // 64, OC)).astype(np.float32))
