@@ -423,7 +423,7 @@ typedef struct qimg_int4_weight {
 } qimg_int4_weight;
 
 /* int4_scratch_bytes (cuda_kernels.cuh:475-487), or more where this
- * library's layout needs it (rank > K/2). */
+ * library's layouts need it (rank > K/2, W4A16 calls of few rows). */
 int64_t qimg_int4_scratch_bytes(int M, int K, int N, int svd_rank);
 
 /* linear_forward_int4 (cuda_kernels.cu:4332-4532): x fp32 [M, K] ->
@@ -431,7 +431,9 @@ int64_t qimg_int4_scratch_bytes(int M, int K, int N, int svd_rank);
  * x / smooth; the low-rank product rounded to bf16) + the residual (W4A16:
  * bf16 of the smoothed, rotated x times the dequantized weight; W4A4:
  * qimg_w4a4_gemm of the INT4-quantized smoothed x) + bias, then GELU-tanh
- * if gelu. scratch >= qimg_int4_scratch_bytes(M, K, N, rank). */
+ * if gelu. scratch >= qimg_int4_scratch_bytes(M, K, N, rank); more changes
+ * nothing. W4A16 also takes less, down to room for the low-rank product in a
+ * GEMM of its own, whose fp32 sums come in another order. */
 int qimg_linear_int4(const float* x, int M, const qimg_int4_weight* w, const uint16_t* bias_bf16, float* out,
                      int gelu, void* scratch, int64_t scratch_bytes, void* stream);
 

@@ -162,8 +162,15 @@ int qimg_w4a4_gemm(const uint8_t* act_packed, const uint8_t* wgt_packed, const f
 
 int64_t qimg_int4_scratch_bytes(int M, int K, int N, int svd_rank) {
     if (M <= 0 || K <= 0 || N <= 0 || svd_rank < 0) return 0;
-    const int64_t mine = std::max(int4_layout(M, K, N, svd_rank, 64, false).total,
-                                  int4_layout(M, K, N, svd_rank, 32, true).total);
+    int64_t mine = std::max(int4_layout(M, K, N, svd_rank, 64, false).total,
+                            int4_layout(M, K, N, svd_rank, 32, true).total);
+    // Room for the extended W4A16 layout at every shape, with the wider of its
+    // steps, so that a buffer of this size or more (one sized for another
+    // layer included) gives a call the same product whatever its capacity.
+    if (svd_rank > 0) {
+        const int pad = (std::min(svd_rank, 256) + 127) / 128 * 128;
+        mine = std::max(mine, int4_ext_layout(M, K, N, svd_rank, pad, true).total);
+    }
     return std::max(mine, reference_int4_scratch(M, K, N, svd_rank));
 }
 
@@ -200,13 +207,20 @@ int qimg_linear_int4(const float* x, int M, const qimg_int4_weight* w, const uin
     uint8_t* base = static_cast<uint8_t*>(scratch);
     uint16_t* xs = reinterpret_cast<uint16_t*>(base + L.xs);
     hipError_t e;
-    // W4A16 with a low-rank branch, whole 128-column stages of K and the room
-    // for it: the low-rank product as `pad` more columns of the residual's (in
+    // W4A16 with a low-rank branch, whole 128-column stages of K and at least
+    // qimg_int4_scratch_bytes of scratch (less, down to the two GEMMs' layout,
+    // is taken too): the low-rank product as `pad` more columns of the residual's (in
     // the same fp32 sums) instead of a GEMM that writes [M, N] and a residual
     // that reads it back. 64 columns a step on the 256x256 tiles, 128 below.
     // 4096 x 3072 x 3072, rank 32: 14 us for the up GEMM and the residual's
-    // accumulate against 2 us for the longer K.
-    if (!w4a4 && r > 0 && qimg::linear_bf16_out16_direct(K, r)) {
+    // accumulate against 2 us for the longer K; whole calls, two GEMMs / one:
+    // 16 rows 36.2 / 32.8 us, 269 x 12288 x 3072 of rank 16 188 / 88, of rank 32
+    // 89.4 / 87.8. Up to 32 rows of a weight wider than long read 4% more
+    // weight for a small [M, N] (12288 x 3072, 16 rows 50.9 / 52.5, 64 rows 54.5
+    // / 54.3) and keep the two GEMMs, where the up GEMM is tiled (r % 32 == 0).
+    const bool joined = !w4a4 && r > 0 && qimg::linear_bf16_out16_direct(K, r) &&
+                        !(M <= 32 && N > 2 * K && r % 32 == 0);
+    if (joined) {
         const int step = qimg::linear_bf16_large(M, K, N) ? 64 : 128;
         const int pad = (r + step - 1) / step * step;
         const Int4ExtLayout X = int4_ext_layout(M, K, N, r, pad, hbs > 1);

@@ -141,3 +141,26 @@ def test_block_wrappers_refuse_operands_of_other_sizes(qimg):
         qimg.mmdit_blocks_forward(None, img, txt, torch.zeros(3071), good)
     with pytest.raises(ValueError, match="float32"):
         qimg.mmdit_blocks_forward(None, img, txt, t_emb, good.double())
+
+
+def test_int4_scratch_bytes_hold_every_w4a16_layout(qimg):
+    """The reported size has room for the W4A16 layout with the low-rank columns
+    beside the input and the weight (up to 128 columns a step), also for a
+    smaller call than the one it was asked for, and is never below the
+    reference's formula."""
+    def a(n):
+        return (n + 255) // 256 * 256
+
+    shapes = [(M, K, N) for M in (1, 16, 132, 512, 4096) for K, N in ((3072, 3072), (3072, 12288), (12288, 3072),
+                                                                      (128, 64))]
+    for M, K, N in shapes:
+        for r in (1, 16, 32, 128, 200, 256):
+            pad = (r + 127) // 128 * 128
+            ext = a(max(N * (K + pad) * 2, r * K * 2)) + a(M * (K + pad) * 2) + a(M * K * 2)
+            got = qimg.int4_scratch_bytes(M, K, N, r)
+            assert got >= ext, (M, K, N, r)
+            ref = a(max(N * K * 2, a(M * (K // 2)) + a(K // 64 * M * 4) + M * N * 4)) + a(M * K * 4) + a(M * K * 2) + \
+                a(M * r * 2)
+            assert got >= ref
+            for m, k, n, rr in ((max(M // 2, 1), K, N, r), (M, K, max(N // 2, 8), r), (M, K, N, max(r // 2, 1))):
+                assert got >= qimg.int4_scratch_bytes(m, k, n, rr)

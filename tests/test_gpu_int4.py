@@ -447,3 +447,24 @@ def test_smooth_hadamard_bit_exact(qimg, oracle, M, K, hbs, smooth):
     np.testing.assert_array_equal(got.cpu().numpy(), ref)
     qimg.smooth_hadamard(xd, _f32(sm) if smooth else None, hbs, out=xd)
     np.testing.assert_array_equal(xd.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("M,N,K,r,hbs", [(1, 3072, 768, 32, 256), (16, 3072, 3072, 16, 1024), (16, 12288, 768, 32, 256),
+                                         (33, 2048, 768, 32, 256), (132, 3072, 3072, 32, 1024),
+                                         (512, 6144, 1024, 32, 1024), (600, 3072, 1024, 32, 1024),
+                                         (5, 1024, 512, 300, 512)])
+def test_linear_w4a16_bits_do_not_depend_on_scratch_capacity(qimg, oracle, M, N, K, r, hbs):
+    """The reported scratch and a far larger buffer give the same bits: few
+    rows, where the wider layout does not fit the reference's formula, among
+    them."""
+    rng = np.random.default_rng(M + N)
+    c = _int4_case(oracle, rng, M, N, K, r, 64, False, True, True, hbs)
+    w = qimg.Int4Weight(N, K, 64, svd_up=_bf16_bits_dev(c["up"]), svd_down=_bf16_bits_dev(c["down"]),
+                        qweight=_u8(c["qw"]), scales4=_f32(c["s4"]), nf4_grid=True, had_block_size=hbs,
+                        smooth=_f32(c["sm"]))
+    x = _f32(c["x"])
+    n = qimg.int4_scratch_bytes(M, K, N, r)
+    out = [qimg.linear_forward_int4(x, w, scratch=torch.empty(size, dtype=torch.uint8, device=DEV))
+           for size in (n, 4 * n + (64 << 20))]
+    torch.cuda.synchronize()
+    assert torch.equal(*out)
