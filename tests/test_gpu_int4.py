@@ -468,3 +468,16 @@ def test_linear_w4a16_bits_do_not_depend_on_scratch_capacity(qimg, oracle, M, N,
            for size in (n, 4 * n + (64 << 20))]
     torch.cuda.synchronize()
     assert torch.equal(*out)
+
+
+@pytest.mark.parametrize("M,N,K,r,gs,hbs,gelu", [
+    (1089, 1030, 256, 300, 64, 256, False),  # rank too wide for the joined product
+    (1089, 1030, 256, 300, 64, 256, True),
+    (1100, 1027, 224, 16, 32, 32, False),    # K not of whole 128
+    (1025, 1028, 96, 16, 32, 32, True),
+    (1025, 1027, 96, 16, 32, 32, False),
+])
+def test_linear_w4a16_short_k_accumulates(qimg, oracle, M, N, K, r, gs, hbs, gelu):
+    """The separate low-rank GEMM's output under the short-K kernel, which reads
+    it back: rows one past a tile, columns past one and not a multiple of 4."""
+    test_linear_int4(qimg, oracle, M, N, K, r, gs, False, True, True, hbs, gelu)
