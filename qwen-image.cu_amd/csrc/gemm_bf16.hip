@@ -653,13 +653,14 @@ hipError_t launch_tiled_bf16(const void* x, int M, int K, const uint16_t* w, int
 template <bool XF32, int TM, int TN>
 hipError_t launch_dma_bf16(const void* x, int M, int K, const uint16_t* w, int N, const uint16_t* bias, float* out,
                            uint16_t* out16, int64_t ldx, int64_t ldo, int gelu, int accumulate, hipStream_t stream) {
+    constexpr int THR = BfDma<XF32, TM, TN>::THR;
     const int tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     if (gelu)
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, true>), dim3(tiles), dim3((BfDma<XF32, TM, TN>::THR)), 0, stream, x, w,
-                           bias, out, out16, ldx, ldo, M, N, K, accumulate);
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, true>), dim3(tiles), dim3(THR), 0, stream, x, w, bias,
+                           out, out16, ldx, ldo, M, N, K, accumulate);
     else
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, false>), dim3(tiles), dim3((BfDma<XF32, TM, TN>::THR)), 0, stream, x, w,
-                           bias, out, out16, ldx, ldo, M, N, K, accumulate);
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<XF32, TM, TN, false>), dim3(tiles), dim3(THR), 0, stream, x, w, bias,
+                           out, out16, ldx, ldo, M, N, K, accumulate);
     return hipGetLastError();
 }
 
@@ -721,9 +722,15 @@ hipError_t launch_linear_bf16(const void* x, int x_dtype, int M, int K, const ui
         return hipGetLastError();
     }
     const int64_t big = static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64);
-    // K of at most 256 (img_in) with enough tiles to fill the chip: no split
-    // of K over the waves
-    if (K <= 256 && big >= 256 && N <= kShortKMaxN) {
+    // K of at most 256 (img_in) and 256 or more tiles of 64x64 (its own 64x128
+    // tiles are half as many): no split of K over the waves. Against the DMA
+    // kernel's K of whole 128 the line is more than 256, its one round of
+    // workgroups (us, fp32 x, DMA / short-K: 300x3072x128 4.4 / 4.4, 342 rows 6.9
+    // / 4.6; 1024x1024x256 5.1 / 5.9, 342x3072x256 7.9 / 6.0, 16384x64x256 5.1 /
+    // 5.5, 32768x64x256 11.5 / 8.3). Against gemm_bf16_kernel it is the faster
+    // form from 64 rows of 3072 on (K = 64: 3.9 / 3.3, 300 rows 9.5 / 3.7, 512
+    // 13.6 / 4.1); below 256 tiles that kernel is kept.
+    if (K <= 256 && big >= (K % 128 == 0 ? 257 : 256) && N <= kShortKMaxN) {
         const int tiles = ((M + SK_M - 1) / SK_M) * ((N + SK_N - 1) / SK_N);
 #define QIMG_SHORTK(XF, GL)                                                                                    \
     hipLaunchKernelGGL((gemm_bf16_shortk_kernel<XF, GL>), dim3(tiles), dim3(BF_THR), 0, stream, x, w, bias, out, M, \

@@ -159,7 +159,8 @@ def test_linear_bf16_rejects_bad_arguments(qimg):
 # stage of K and fewer stages than the ring holds; short K on 64 x 128 tiles
 DMA = [(1, 1, 128), (17, 61, 128), (15, 33, 256), (65, 4097, 384), (129, 6145, 512), (1025, 67, 3072),
        (4097, 32, 1152), (300, 3074, 3584), (1000, 3000, 1024), (4096, 16, 3072), (16385, 64, 256),
-       (1025, 3075, 64), (4095, 1027, 32), (2049, 2051, 224)]
+       (1025, 3075, 64), (4095, 1027, 32), (2049, 2051, 224), (1021, 1023, 128), (1025, 1023, 128),
+       (16384, 64, 256)]
 
 
 @pytest.mark.parametrize("M,N,K", DMA)
