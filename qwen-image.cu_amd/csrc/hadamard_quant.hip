@@ -894,7 +894,8 @@ __global__ __launch_bounds__(256) void smooth_fwht_wave_rows_kernel(const float*
 #pragma unroll
     for (int b = 0; b < NB; ++b)
         smooth_chunk(x + base, smooth, static_cast<uint16_t*>(nullptr), b * (HBS / 16) + lane, v[b]);
-    wave_row_fwht_store<RowOut::Bf16, NB>(v, lds, lane, row, K, norm, Bf16Dest{xs != nullptr ? xs + base : nullptr, xr});
+    const Bf16Dest dst{xs != nullptr ? xs + base : nullptr, xr};
+    wave_row_fwht_store<RowOut::Bf16, NB>(v, lds, lane, row, K, norm, dst);
     for (int i = lane; i < pad / 8; i += 64) reinterpret_cast<u32x4*>(xr + K)[i] = (u32x4){0u, 0u, 0u, 0u};
 }
 

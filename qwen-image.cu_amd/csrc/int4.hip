@@ -8,8 +8,8 @@
 // v_mfma_i32_32x32x32_i8: a 32-bit word of eight nibbles becomes two words of
 // int8 lanes with one AND each, (w << 4) & 0xF0F0F0F0 and w & 0xF0F0F0F0: each
 // byte is 16 x the signed nibble (two's complement in the high half of the
-// byte), so the MFMA returns 256 x the exact dot product, and an arithmetic
-// shift by 8 recovers it. The element order inside a fragment is a
+// byte), so the MFMA returns 256 x the exact dot product, and the 2^-8 goes
+// into the activation scale. The element order inside a fragment is a
 // permutation of k that is the same for both operands, so every dot product
 // is the exact int32 sum of the reference's group. Each group's sum is then
 // rescaled and accumulated in fp32 in the reference's operation order,
@@ -42,8 +42,9 @@ __device__ __forceinline__ float int4_code(int n, int nf4, int signed_int4) {
 // parts by rows, cost the long rows 0.2 us.)
 constexpr int ROW_THR = 128, SHORT_THR = 256;
 struct RowThread {
-    int row, sub, col, step;  // the thread's first row (its sub-th of the workgroup's), its place in it, rows to the next
-    bool live;                // false: past the last of the rpw rows
+    int row, sub;   // the thread's first row, and which of the workgroup's rows that is
+    int col, step;  // its place in the row, and rows to the next one
+    bool live;      // false: past the last of the rpw rows
 };
 template <bool SHORT, int THR>
 __device__ __forceinline__ RowThread row_thread(int per, int nb) {
@@ -72,7 +73,8 @@ __global__ __launch_bounds__(SHORT ? SHORT_THR : ROW_THR) void dequant_int4_bf16
                                                                 const float* __restrict__ scales,
                                                                 uint16_t* __restrict__ out, int N, int K, int gs,
                                                                 int nf4, int scales_gn, int signed_int4,
-                                                                const uint16_t* __restrict__ up, int r, int pad, int nb) {
+                                                                const uint16_t* __restrict__ up, int r, int pad,
+                                                                int nb) {
     __shared__ float2 table[256];
     for (int i = threadIdx.x; i < 256; i += SHORT ? SHORT_THR : ROW_THR)
         table[i] = make_float2(int4_code(i & 15, nf4, signed_int4), int4_code(i >> 4, nf4, signed_int4));
@@ -259,17 +261,21 @@ __global__ __launch_bounds__(SHORT || V == 2 ? 256 : ROW_THR) void quant_act_int
 // The kernel is bound by the vector ALU: each group of 64 columns costs a
 // 32 x 32 block two MFMAs (64 cycles of the matrix core) and 16 x 4 vector
 // operations (a conversion, two products and a sum per accumulator in the
-// reference's rounding order, 256 cycles). So everything else is kept off the
-// vector pipe's critical path: packed operands come by DMA into a two-slot
-// LDS ring of 128 columns (one barrier a stage), and the outputs are laid out
-// with n across the lanes, so a store writes 128 consecutive bytes of two rows
-// and the activation scales are LDS broadcasts. A wave owns 32 x 64 outputs
-// (four waves per SIMD); 64 x 64 (two per SIMD, fewer unpacks per product)
-// measured 134 against 112 us at 4352 x 3072 x 3072, group 64, and 48 against
-// 30 us at 256 rows. Before, lanes ran across m (each 4-byte access touched
-// 64 lines) and fragments were loaded straight from global memory: 254 us, and
-// 19 us more for the low-rank product that is now multiplied here. 112 us is
-// 0.73 POP/s; the vector operations alone take about 92 us.
+// reference's rounding order, 256 cycles), to which the compiled code of groups
+// of 64 and 128 adds a copy of each MFMA result out of the accumulation
+// registers (16 operations) and about 23 of unpacking and addressing: 415 in the
+// loop of a stage of 2 x 2 groups and blocks, 106 us at 4352 x 3072 x 3072, group
+// 64, and 2.4 GHz (the 16 x 4 alone: 65). So everything else is kept off the
+// vector pipe's critical path: packed operands come by DMA into a two-slot LDS
+// ring of 128 columns (one barrier a stage), and the outputs are laid out with n
+// across the lanes, so a store writes 128 consecutive bytes of two rows and the
+// activation scales are LDS broadcasts. A wave owns 32 x 64 outputs (four waves
+// per SIMD; three for groups of 128, which hold 140 registers); 64 x 64 (two per
+// SIMD, fewer unpacks per product) measured 134 against 112 us at 4352 x 3072 x
+// 3072, group 64, and 48 against 30 us at 256 rows. Before, lanes ran across m
+// (each 4-byte access touched 64 lines) and fragments were loaded straight from
+// global memory: 254 us, and 19 us more for the low-rank product that is now
+// multiplied here. 112 us is 0.73 POP/s.
 constexpr int W4_THR = 256;   // four waves, 2 x 2
 constexpr int W4_BM = 64;
 constexpr int W4_BN = 128;
@@ -542,13 +548,16 @@ __global__ __launch_bounds__(256) void awq_dequant_kernel(const int32_t* __restr
 
 // awq_gemv_repacked_kernel (cuda_kernels.cu:3106-3153), M = 1, gs = 64. The
 // sum over ic runs in order, so each output channel is one dependent chain of
-// IC additions, and a wave cannot issue a dependent addition before 8.4 cycles
-// have passed: 3072 of them are 11 us. Everything else is taken off that chain.
-// A workgroup owns 64 channels, one per lane: eight waves load the weight words
-// AWQ_DEPTH stages ahead, form the products and put them in a two-slot LDS
-// ring of 128 inputs; a ninth wave, first in the issue order, reads them (16
-// bytes a lane, the next 32 inputs while it adds the last) and adds. q * s is exact in fp32 (4 bits x a
-// bf16's 8), so fma(q, s, z) is the reference's q * s + z.
+// IC additions, and a dependent v_add_f32 takes 8.25 cycles: 3072 of them are
+// 10.6 us at 2.4 GHz. Everything else is taken off that chain. A workgroup
+// owns 64 channels, one per lane: eight waves load the weight words, form the
+// products and put them in a two-slot LDS ring of 128 inputs; a ninth wave, first
+// in the issue order, reads them (16 bytes a lane, the next 32 inputs while it
+// adds the last) and adds. From the second stage on the words are loaded
+// AWQ_DEPTH stages ahead; the compiler sinks the first loads below the barrier
+// that x waits for, which the ninth wave copies alone, so a launch starts with
+// both latencies in a row. q * s is exact in fp32 (4 bits x a bf16's 8), so
+// fma(q, s, z) is the reference's q * s + z.
 // 18432 x 3072 (32 MB of weights and scales): 22.4 us; one wave per 64 channels
 // doing all of it took 74.6. With x in scalar registers, whose load latency
 // falls on every stage's barrier, 32.7; with the last sums' operands read in

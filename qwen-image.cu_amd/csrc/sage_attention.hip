@@ -57,9 +57,11 @@ __host__ __device__ constexpr int div_up(int a, int b) { return (a + b - 1) / b;
 // measured faster than 16, whose loads touch 32 rows for 32 bytes each,
 // and than 64). Wave 0 only
 // sums, one chain per lane (lanes past KM_DIMS repeat a chain and store
-// nothing), one fp32 add per token (the fp16 -> fp32 conversions stay off
-// the dependent chain), with the LDS reads of each group of 32 tokens
-// issued two groups ahead. Waves 1-3
+// nothing), one fp32 add per token; the fp16 -> fp32 conversions are not on the
+// dependent chain, but are a second instruction per token of the same wave. It
+// reads 64 tokens at a time from LDS: the source reads two groups of 32 two
+// groups ahead, the compiled loop issues both groups' reads after the adds of
+// the last one and waits for them a few conversions into the next. Waves 1-3
 // stream chunks of k[h, :, d0:d0+32] (each lane 16 bytes =
 // 8 dims of 4 consecutive tokens), transpose 4 tokens x 8 dims in registers
 // and store them to LDS as [d][s] with 8-byte writes; rows are padded to a
@@ -165,8 +167,7 @@ __device__ __forceinline__ void k_mean_slice(const uint16_t* __restrict__ k, flo
             const int n = min(CHUNK, S - c * CHUNK);
             const uint32_t* row = &tile[(buf * KM_DIMS + lane % KM_DIMS) * PITCH];
             auto rd = [&](int t8) { return *reinterpret_cast<const u32x4*>(row + 4 * t8); };
-            // groups of 32 tokens, read two groups ahead in two register
-            // sets; a read past the chunk's last full group re-reads group
+            // groups of 32 tokens in two register sets; a read past the chunk's last full group re-reads group
             // 0 (in bounds, unused)
             const int full = n >> 5;
             auto group = [&](int gi, u32x4 (&cur)[4]) {

@@ -249,7 +249,8 @@ def test_quant_repeatable_and_empty(qimg):
     assert e[0].shape == (0, 3072)
 
 
-@pytest.mark.parametrize("K,hbs", [(2048, 1024), (3072, 1024), (4096, 1024), (8192, 4096), (12288, 4096), (16384, 4096)])
+@pytest.mark.parametrize("K,hbs", [(2048, 1024), (3072, 1024), (4096, 1024), (8192, 4096), (12288, 4096),
+                                   (16384, 4096)])
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_quant_rows_do_not_depend_on_their_number(qimg, K, hbs, fp8, bf16):
