@@ -466,7 +466,10 @@ __global__ __launch_bounds__(256) void v_relayout_kernel(const uint16_t* __restr
 // x 128 273.3 -> 252.7 us (mean 27 + Q 12 + V 9.6 before), 24 x 1301 64.6 ->
 // 55.2 us. The mean's chunk is 512 tokens (66 KB of LDS) instead of 1024
 // (132 KB), so that two workgroups share a CU and its first chunk arrives
-// sooner; 256 measured 254.7 and 55.0 us.
+// sooner; 256 measured 254.7 and 55.0 us. Over other sizes the call gains or is
+// equal, also where the two passes lose waves to the mean's LDS: 1 x 77 20.1 ->
+// 14.2 us, 1000 x 77 115 -> 82, 4000 x 64 330 -> 232, 96 x 1024 110 -> 97, 48 x
+// 4352 525 -> 515, 48 x 7401 1254 -> 1245.
 constexpr int PREP_CHUNK = 512;
 template <int D>
 __global__ __launch_bounds__(256) void sage_prep_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
